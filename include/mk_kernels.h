@@ -205,8 +205,9 @@ int mk_gemm_bf16_nt(const void* a, const void* bt, void* c, const void* aux, int
  *               (K <= 128, bf16 output, no paired epilogue)
  *   SHORT       128 x 128 with all of K in LDS (M, N % 128, K % 32,
  *               K <= 256, bf16 output, no paired epilogue)
- *   REG256      256 x 256, register-staged operands (M, N % 256, K % 64)
- *   GENERIC256, GENERIC128  any shape (no paired epilogue)
+ *   T16x64 .. T256x256  tiles of that size, any shape (no paired epilogue)
+ *   REG256      another name of T256x256 (M, N % 256, K % 64)
+ *   GENERIC256, GENERIC128  other names of T256x256 and T128x128
  * The reference picks between its GEMM variants the same way, by timing
  * them at the first plan build and keeping the fastest per device and
  * shape (AutotuneGemm, src/pjrt_plugin/core/mps_executable.mm:3433-3725;
@@ -220,7 +221,13 @@ enum {
   MK_GEMM_ROUTE_REG256 = 5,
   MK_GEMM_ROUTE_GENERIC256 = 6,
   MK_GEMM_ROUTE_GENERIC128 = 7,
-  MK_GEMM_ROUTE_COUNT = 8
+  MK_GEMM_ROUTE_T16x64 = 16,
+  MK_GEMM_ROUTE_T32x64 = 17,
+  MK_GEMM_ROUTE_T64x64 = 18,
+  MK_GEMM_ROUTE_T128x64 = 19,
+  MK_GEMM_ROUTE_T128x128 = 20,
+  MK_GEMM_ROUTE_T256x256 = 21,
+  MK_GEMM_ROUTE_COUNT = 22  /* 8 .. 15 name no route */
 };
 
 /* mk_gemm_bf16_epilogue (epilogue MK_EPI_NONE: mk_gemm_bf16, with
@@ -272,14 +279,15 @@ const char* mk_gemm_autotune_header(void);
  *   - K == 1 is a plain product, keeping XLA's signed zero (:904-1004);
  *   - any K and N, operands read through element strides (a transposed
  *     operand or a vector needs no copy);
- *   - F32 / BF16 / F16 inputs accumulate in f32 in k order; the result is
- *     F32 or the input type (round to nearest even).
+ *   - F32 / BF16 / F16 inputs accumulate in f32; the result is F32 or the
+ *     input type (round to nearest even).
  * C[b, m, n] = sum_k A[b, m, k] B[b, k, n]; A[b, m, k] is element
  * b*a_strides[0] + m*a_strides[1] + k*a_strides[2] of a, B[b, k, n] element
  * b*b_strides[0] + k*b_strides[1] + n*b_strides[2] of b; C is contiguous
  * [batch, M, N].  Types use the PJRT_Buffer_Type numbering below; both
- * operands must have the same type (MK_EUNSUPPORTED otherwise).  One
- * thread per output element: not a throughput path. */
+ * operands must have the same type (MK_EUNSUPPORTED otherwise).  bf16 and
+ * f16 operands with one contiguous dimension each run on the matrix cores
+ * from K = 16; the rest has one thread per output element. */
 enum {
   MK_TYPE_S8 = 2, MK_TYPE_S16 = 3, MK_TYPE_S32 = 4, MK_TYPE_S64 = 5, MK_TYPE_U8 = 6, MK_TYPE_U16 = 7,
   MK_TYPE_U32 = 8, MK_TYPE_U64 = 9, MK_TYPE_F16 = 10, MK_TYPE_F32 = 11, MK_TYPE_BF16 = 13

@@ -42,6 +42,7 @@ KERNEL_SOURCES = [
     "kernels/qgemm.hip",
     "kernels/decoder.hip",
     "kernels/gemm.hip",
+    "kernels/gemm_tile.hip",
     "kernels/dot_general.hip",
     "kernels/rowops.hip",
     "kernels/eltwise.hip",

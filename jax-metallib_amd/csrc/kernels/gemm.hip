@@ -7,25 +7,16 @@
 //   (preferred_element_type = f32 returns f32, binary_ops.mm:775-782)
 // f32  x f32  -> f32 (v_mfma_f32_16x16x4_f32, full f32 products)
 //
-// Design:
-//   * Block tile BM x BN x 64 (bf16) with WM x WN waves; every wave owns a
-//     (BM/WM) x (BN/WN) sub-tile of 16x16 MFMA tiles held in accumulators.
-//   * Global -> registers -> LDS double buffering, one barrier per k-tile:
-//     the next k-tile's global loads are in flight while the MFMAs consume
-//     the current one.
-//   * A is staged as-is ([m][k], k contiguous).  B arrives n-contiguous, but
-//     the MFMA wants k runs per lane, so each thread transposes an 8x8 block
-//     of B in registers (v_perm_b32 on 16-bit halves) while staging; LDS then
-//     holds B as [n][k].  Rows are padded to 144 B so the 16-byte fragment
-//     reads of 16 consecutive rows hit distinct LDS banks.
-//   * The MFMA is issued as B-fragment x A-fragment, which yields C^T tiles:
-//     each lane then owns 4 consecutive columns of one row, stored as one
-//     8-byte (bf16) or 16-byte (f32) write.
-//   * Workgroup -> tile mapping is XCD-aware: runs of consecutive logical
-//     ids stay on one XCD and cover a 4-row band of tiles, so the A panels and
-//     B panels they share stay in that XCD's L2.
+// The bf16 kernels here take M and N in multiples of 256 (128 for the
+// short-K one); gemm_tile.hip takes every other shape, and these where its
+// smaller tiles fill the chip better.  The MFMA is issued as B-fragment x
+// A-fragment, which yields C^T tiles: each lane then owns 4 consecutive
+// columns of one row.  Workgroup -> tile mapping is XCD-aware: runs of
+// consecutive logical ids stay on one XCD and cover a 4-row band of tiles, so
+// the A panels and B panels they share stay in that XCD's L2.
 #include "common.h"
 #include "epilogue.h"
+#include "gemm_tile.h"
 
 namespace mk {
 
@@ -40,12 +31,6 @@ struct GemmArgs {
   const uint16_t* aux; // bf16, same layout and batch stride as C
 };
 
-// Four bf16 outputs of C row-major at offset off, with the GEMM's epilogue.
-__device__ __forceinline__ void store_bf16x4(const GemmArgs& p, uint16_t* C, const uint16_t* X, size_t off,
-                                             const f32x4& acc) {
-  epi_store_bf16x4(C, X, p.epi, off, acc);
-}
-
 // Map a logical workgroup id to a (tile row, tile col) with bands of GM tile
 // rows, so consecutive ids sweep a GM-tall column block.
 __device__ __forceinline__ void tile_coords(uint32_t L, int tiles_m, int tiles_n, int& tm, int& tn) {
@@ -58,157 +43,6 @@ __device__ __forceinline__ void tile_coords(uint32_t L, int tiles_m, int tiles_n
   } else {
     tm = (int)L / tiles_n;
     tn = (int)L - tm * tiles_n;
-  }
-}
-
-template <int BM, int BN, int WM, int WN>
-__global__ __launch_bounds__(WM * WN * 64) void gemm_bf16_kernel(GemmArgs p) {
-  constexpr int BK = 64;
-  constexpr int LDK = BK + 8;  // padded row length (bf16 elements)
-  constexpr int NT = WM * WN * 64;
-  constexpr int TM = BM / WM / 16;
-  constexpr int TN = BN / WN / 16;
-  constexpr int ACH = BM * BK / 8 / NT;             // A 16-byte chunks per thread
-  constexpr int BTOT = (BK / 8) * (BN / 8);         // B 8x8 blocks per tile
-  constexpr int BBL = (BTOT + NT - 1) / NT;         // B blocks per thread
-  static_assert(ACH * NT * 8 == BM * BK, "A staging must divide evenly");
-
-  extern __shared__ __align__(16) unsigned char smem[];
-  uint16_t* As = reinterpret_cast<uint16_t*>(smem);  // [2][BM][LDK]
-  uint16_t* Bs = As + 2 * BM * LDK;                   // [2][BN][LDK]
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave / WN, wn = wave % WN;
-  const int tiles_m = (p.M + BM - 1) / BM, tiles_n = (p.N + BN - 1) / BN;
-  int tm, tn;
-  tile_coords(xcd_logical_id(blockIdx.x, gridDim.x), tiles_m, tiles_n, tm, tn);
-  const int m0 = tm * BM, n0 = tn * BN;
-  const uint16_t* A = static_cast<const uint16_t*>(p.a) + (size_t)blockIdx.z * p.sa;
-  const uint16_t* B = static_cast<const uint16_t*>(p.b) + (size_t)blockIdx.z * p.sb;
-  const int M = p.M, N = p.N, K = p.K;
-
-  u32x4 ra[ACH];
-  u32x4 rb[BBL][8];
-
-  auto load_tile = [&](int k0) {
-#pragma unroll
-    for (int i = 0; i < ACH; ++i) {
-      const int q = tid + i * NT;
-      const int row = q / (BK / 8), kc = q % (BK / 8);
-      const int gm = m0 + row, gk = k0 + 8 * kc;
-      ra[i] = (gm < M && gk < K) ? *reinterpret_cast<const u32x4*>(A + (size_t)gm * K + gk)
-                                 : u32x4{0u, 0u, 0u, 0u};
-    }
-#pragma unroll
-    for (int i = 0; i < BBL; ++i) {
-      const int q = tid + i * NT;
-      const int kb = q / (BN / 8), nb = q % (BN / 8);
-      const int gn = n0 + 8 * nb;
-#pragma unroll
-      for (int r = 0; r < 8; ++r) {
-        const int gk = k0 + 8 * kb + r;
-        rb[i][r] = (q < BTOT && gn < N && gk < K) ? *reinterpret_cast<const u32x4*>(B + (size_t)gk * N + gn)
-                                      : u32x4{0u, 0u, 0u, 0u};
-      }
-    }
-  };
-
-  auto store_tile = [&](int buf) {
-    uint16_t* as = As + buf * BM * LDK;
-    uint16_t* bs = Bs + buf * BN * LDK;
-#pragma unroll
-    for (int i = 0; i < ACH; ++i) {
-      const int q = tid + i * NT;
-      const int row = q / (BK / 8), kc = q % (BK / 8);
-      *reinterpret_cast<u32x4*>(as + row * LDK + 8 * kc) = ra[i];
-    }
-#pragma unroll
-    for (int i = 0; i < BBL; ++i) {
-      const int q = tid + i * NT;
-      if (q >= BTOT) break;
-      const int kb = q / (BN / 8), nb = q % (BN / 8);
-      // Transpose the 8 (k) x 8 (n) block: column c gets halfword c of rows 0..7.
-      const uint32_t* w = reinterpret_cast<const uint32_t*>(&rb[i][0]);
-#pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        const uint32_t sel = (c & 1) ? 0x07060302u : 0x05040100u;
-        const int d = c >> 1;
-        u32x4 o;
-        o.x = perm(w[1 * 4 + d], w[0 * 4 + d], sel);
-        o.y = perm(w[3 * 4 + d], w[2 * 4 + d], sel);
-        o.z = perm(w[5 * 4 + d], w[4 * 4 + d], sel);
-        o.w = perm(w[7 * 4 + d], w[6 * 4 + d], sel);
-        *reinterpret_cast<u32x4*>(bs + (8 * nb + c) * LDK + 8 * kb) = o;
-      }
-    }
-  };
-
-  f32x4 acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  const int KT = (K + BK - 1) / BK;
-  load_tile(0);
-  store_tile(0);
-  __syncthreads();
-
-  const int arow = wm * TM * 16 + (lane & 15);
-  const int brow = wn * TN * 16 + (lane & 15);
-  const int kofs = 8 * (lane >> 4);
-
-  for (int kt = 0; kt < KT; ++kt) {
-    const int buf = kt & 1;
-    if (kt + 1 < KT) load_tile((kt + 1) * BK);
-    const uint16_t* as = As + buf * BM * LDK;
-    const uint16_t* bs = Bs + buf * BN * LDK;
-#pragma unroll
-    for (int ks = 0; ks < BK / 32; ++ks) {
-      u32x4 af[TM], bf[TN];
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-        af[i] = *reinterpret_cast<const u32x4*>(as + (arow + 16 * i) * LDK + 32 * ks + kofs);
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-        bf[j] = *reinterpret_cast<const u32x4*>(bs + (brow + 16 * j) * LDK + 32 * ks + kofs);
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = mfma16x16x32(bf[j], af[i], acc[i][j]);
-    }
-    if (kt + 1 < KT) store_tile(buf ^ 1);
-    __syncthreads();
-  }
-
-  // Epilogue: lane owns row m, columns n..n+3 of each 16x16 tile.
-  const int mrow = m0 + wm * TM * 16 + (lane & 15);
-  const int ncol = n0 + wn * TN * 16 + 4 * (lane >> 4);
-  if (p.out_f32) {
-    float* C = static_cast<float*>(p.c) + (size_t)blockIdx.z * p.sc;
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      const int m = mrow + 16 * i;
-      if (m >= M) continue;
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int n = ncol + 16 * j;
-        if (n < N) *reinterpret_cast<f32x4*>(C + (size_t)m * N + n) = acc[i][j];
-      }
-    }
-  } else {
-    uint16_t* C = static_cast<uint16_t*>(p.c) + (size_t)blockIdx.z * p.sc;
-    const uint16_t* X = p.aux + (p.epi != MK_EPI_NONE ? (size_t)blockIdx.z * p.sc : 0);
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      const int m = mrow + 16 * i;
-      if (m >= M) continue;
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int n = ncol + 16 * j;
-        if (n < N) store_bf16x4(p, C, X, (size_t)m * N + n, acc[i][j]);
-      }
-    }
   }
 }
 
@@ -352,151 +186,12 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_f32_kernel(GemmArgs p) {
 }
 
 
-// ---------------------------------------------------------------------------
-// Large-tile bf16 GEMM (M % 256 == 0, N % 256 == 0, K % 64 == 0).
-//
-// 256 x 256 x 64 workgroup tile; WM x WN waves (2 x 4: each wave a 128 x 64
-// tile of 8 x 4 16x16x32 MFMA accumulators; 2 x 2: 128 x 128, 8 x 8).  Both operands are
-// staged in LDS in their natural layouts (A [m][k], B [k][n]) through
-// registers with one barrier per k-tile (double buffer, 128 KB).  The B
-// fragments come straight out of the [k][n] layout with gfx950's transposing
-// LDS read, ds_read_b64_tr_b16: within each 16-lane group, lanes 4r + q name
-// the 8 bytes of row r, columns 4q..4q+3, and lane j receives column j of
-// the 4 x 16 block -- four consecutive k of one n, i.e. half of an MFMA
-// fragment.  No register transposes remain.
-//
-// LDS swizzles (16-byte chunks): A row r, chunk c lives at chunk
-// c ^ ((r >> 1) & 7), so the 16 rows of one fragment read cover all 64
-// banks; B row k, chunk c lives at c ^ (k & 3 | ((k >> 3) & 3) << 2), so the
-// 16 rows one transposing read touches land in 16 different 16-byte slots.
-// ---------------------------------------------------------------------------
+// gfx950's transposing LDS read, ds_read_b64_tr_b16: within each 16-lane
+// group, lanes 4r + q name the 8 bytes of row r, columns 4q..4q+3 of a
+// [k][n] tile, and lane j receives column j of the 4 x 16 block -- four
+// consecutive k of one n, half of an MFMA fragment.
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4* lds_s16x4_ptr;
-
-__device__ __forceinline__ int swz_a(int row, int c) { return c ^ ((row >> 1) & 7); }
-__device__ __forceinline__ int swz_b(int k, int c) { return c ^ ((k & 3) | (((k >> 3) & 3) << 2)); }
-
-__device__ __forceinline__ u32x2 lds_tr16(const uint16_t* p) {
-  const s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(p));
-  return __builtin_bit_cast(u32x2, v);
-}
-
-template <int WM_, int WN_>
-__global__ __launch_bounds__(WM_ * WN_ * 64) void gemm_bf16_256_kernel(GemmArgs p) {
-  constexpr int BM = 256, BN = 256, BK = 64, NT = WM_ * WN_ * 64;
-  constexpr int TM = BM / WM_ / 16, TN = BN / WN_ / 16;  // per-wave MFMA tiles
-  constexpr int CH = BM * BK / 8 / NT;                   // 16-byte chunks per thread (A and B each)
-  extern __shared__ __align__(16) unsigned char smem[];
-  uint16_t* As = reinterpret_cast<uint16_t*>(smem);  // [2][BM * BK]
-  uint16_t* Bs = As + 2 * BM * BK;                    // [2][BK * BN]
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave / WN_, wn = wave % WN_;
-  const int tiles_m = p.M / BM, tiles_n = p.N / BN;
-  int tm, tn;
-  tile_coords(xcd_logical_id(blockIdx.x, gridDim.x), tiles_m, tiles_n, tm, tn);
-  const int m0 = tm * BM, n0 = tn * BN;
-  const uint16_t* A = static_cast<const uint16_t*>(p.a) + (size_t)blockIdx.z * p.sa + (size_t)m0 * p.K;
-  const uint16_t* B = static_cast<const uint16_t*>(p.b) + (size_t)blockIdx.z * p.sb + n0;
-  const int K = p.K, N = p.N;
-
-  // Staging: CH A chunks (row q/8, chunk q%8) and CH B chunks (row q/32,
-  // chunk q%32) per thread, q = tid + NT * i, moved in two halves so only
-  // CH/2 + CH/2 chunks sit in registers at a time: half h of the next tile is
-  // loaded before 32-k step h and stored to the free buffer after it.
-  constexpr int HC = CH / 2;
-  static_assert(HC * 2 == CH, "staging splits in halves");
-  u32x4 ra[HC], rb[HC];
-  auto load_half = [&](int k0, int h) {
-#pragma unroll
-    for (int i = 0; i < HC; ++i) {
-      const int q = tid + NT * (h * HC + i);
-      ra[i] = *reinterpret_cast<const u32x4*>(A + (size_t)(q >> 3) * K + k0 + 8 * (q & 7));
-      rb[i] = *reinterpret_cast<const u32x4*>(B + (size_t)(k0 + (q >> 5)) * N + 8 * (q & 31));
-    }
-  };
-  auto store_half = [&](int buf, int h) {
-    uint16_t* as = As + buf * BM * BK;
-    uint16_t* bs = Bs + buf * BK * BN;
-#pragma unroll
-    for (int i = 0; i < HC; ++i) {
-      const int q = tid + NT * (h * HC + i);
-      const int ar = q >> 3, ac = q & 7, br = q >> 5, bc = q & 31;
-      *reinterpret_cast<u32x4*>(as + ar * BK + 8 * swz_a(ar, ac)) = ra[i];
-      *reinterpret_cast<u32x4*>(bs + br * BN + 8 * swz_b(br, bc)) = rb[i];
-    }
-  };
-
-  f32x4 acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  const int KT = K / BK;
-  load_half(0, 0);
-  store_half(0, 0);
-  load_half(0, 1);
-  store_half(0, 1);
-  __syncthreads();
-
-  // Per-lane fragment coordinates.
-  const int arow0 = wm * (16 * TM) + (lane & 15);   // + 16 * i
-  const int akb = lane >> 4;                          // k block (8 k) in a 32-k step
-  const int g = lane >> 4, r = (lane & 15) >> 2, q = lane & 3;
-  const int bcol0 = wn * (16 * TN) + 4 * q;          // + 16 * j
-
-  for (int kt = 0; kt < KT; ++kt) {
-    const int buf = kt & 1;
-    const bool more = kt + 1 < KT;
-    const uint16_t* as = As + buf * BM * BK;
-    const uint16_t* bs = Bs + buf * BK * BN;
-#pragma unroll
-    for (int ks = 0; ks < BK / 32; ++ks) {
-      if (more) load_half((kt + 1) * BK, ks);
-      // All B fragments of the step, then one A fragment per row of tiles
-      // (keeps only TN + 1 fragments live).
-      u32x4 bf[TN];
-      const int k1 = 32 * ks + 8 * g + r;
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int col = bcol0 + 16 * j;
-        const u32x2 lo = lds_tr16(bs + k1 * BN + 8 * swz_b(k1, col >> 3) + (col & 7));
-        const u32x2 hi = lds_tr16(bs + (k1 + 4) * BN + 8 * swz_b(k1 + 4, col >> 3) + (col & 7));
-        bf[j] = u32x4{lo.x, lo.y, hi.x, hi.y};
-      }
-#pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        const int row = arow0 + 16 * i;
-        const u32x4 af = *reinterpret_cast<const u32x4*>(as + row * BK + 8 * swz_a(row, 4 * ks + akb));
-#pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = mfma16x16x32(bf[j], af, acc[i][j]);
-      }
-      if (more) store_half(buf ^ 1, ks);
-    }
-    __syncthreads();
-  }
-
-  // Epilogue (C^T tiles): lane owns row m, columns n..n+3 of each tile.
-  const int mrow = m0 + wm * (16 * TM) + (lane & 15);
-  const int ncol = n0 + wn * (16 * TN) + 4 * (lane >> 4);
-  if (p.out_f32) {
-    float* C = static_cast<float*>(p.c) + (size_t)blockIdx.z * p.sc;
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-        *reinterpret_cast<f32x4*>(C + (size_t)(mrow + 16 * i) * N + ncol + 16 * j) = acc[i][j];
-  } else {
-    uint16_t* C = static_cast<uint16_t*>(p.c) + (size_t)blockIdx.z * p.sc;
-    const uint16_t* X = p.aux + (p.epi != MK_EPI_NONE ? (size_t)blockIdx.z * p.sc : 0);
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) store_bf16x4(p, C, X, (size_t)(mrow + 16 * i) * N + ncol + 16 * j, acc[i][j]);
-  }
-}
-
 
 // ---------------------------------------------------------------------------
 // 256 x 256 tile fed by LDS DMA.
@@ -1176,18 +871,6 @@ hipError_t lds_opt_in(const void* fn, size_t bytes) {
 }
 
 template <int BM, int BN, int WM, int WN>
-hipError_t launch_bf16(const mk::GemmArgs& a, int batch, hipStream_t st) {
-  constexpr size_t lds = (size_t)2 * (BM + BN) * (64 + 8) * 2;
-  const void* fn = (const void*)mk::gemm_bf16_kernel<BM, BN, WM, WN>;
-  hipError_t e = lds_opt_in(fn, lds);
-  if (e != hipSuccess) return e;
-  const int tiles = ((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN);
-  hipLaunchKernelGGL((mk::gemm_bf16_kernel<BM, BN, WM, WN>), dim3(tiles, 1, batch),
-                     dim3(WM * WN * 64), lds, st, a);
-  return hipGetLastError();
-}
-
-template <int BM, int BN, int WM, int WN>
 hipError_t launch_f32(const mk::GemmArgs& a, int batch, hipStream_t st) {
   constexpr size_t lds = (size_t)2 * (BM + BN) * (32 + 4) * 4;
   const void* fn = (const void*)mk::gemm_f32_kernel<BM, BN, WM, WN>;
@@ -1242,6 +925,11 @@ int env_tile() {
 
 namespace {
 
+bool route_known(int route) {
+  return (route > MK_GEMM_ROUTE_DEFAULT && route <= MK_GEMM_ROUTE_GENERIC128) ||
+         (route >= MK_GEMM_ROUTE_T16x64 && route <= MK_GEMM_ROUTE_T256x256);
+}
+
 // bt: b is B^T [N, K] (only the DMA-fed 256 x 256 kernel takes it).
 // Routes: the kernel choices of the [K, N] bf16 product (MK_GEMM_ROUTE_*).
 // Every route computes each output's k in the same order in the same MFMA,
@@ -1264,64 +952,80 @@ bool route_fits(int route, int64_t M, int64_t N, int64_t K, int epi, int out_f32
     case MK_GEMM_ROUTE_GENERIC128:
       return simple_epi;
     default:
-      return false;
+      return route >= MK_GEMM_ROUTE_T16x64 && route <= MK_GEMM_ROUTE_T256x256 && simple_epi;
   }
+}
+
+// The packed product as the tile family takes it.
+mkg::TileGemm tile_args(const mk::GemmArgs& p, int64_t batch, bool bt = false) {
+  const char* dma_env = getenv("MK_GEMM_DMA");
+  mkg::TileGemm g;
+  g.registers = dma_env && dma_env[0] == '0';
+  g.a = p.a;
+  g.b = p.b;
+  g.c = p.c;
+  g.aux = p.aux;
+  g.batch = batch;
+  g.M = p.M;
+  g.N = p.N;
+  g.K = p.K;
+  g.lda = p.K;
+  g.ldb = bt ? p.K : p.N;
+  g.b_t = bt;
+  g.sa = p.sa;
+  g.sb = p.sb;
+  g.out_f32 = p.out_f32 != 0;
+  g.epi = p.epi;
+  return g;
 }
 
 // The built-in choice (what MK_GEMM_* environment knobs steer), from
 // timings with operands rotated past the 256 MB Infinity Cache (one box,
 // us):
-//   - K >= 512 on 256-multiples: the pipelined kernel (fragment prefetch,
-//     5-stage ring) at any tile count: 2048^3 51.1 against 54.2 (128-tile
-//     kernel) / 58.6 (ring); 1024^3 28.4 / 28.6 / 31.8; 16 x 1024^3 42.9 /
-//     77.3 / 45.2; 8192^2 x 1024 151.6 / 288.2 / 153.4; 256 x 14336 x 4096
-//     102.1 / 103.5 / 106.7 (8 x 512^2 x 4096: 106.4 / 103.7 / 114.0).  It
-//     runs at a lower clock (GRBM_GUI_ACTIVE per ns ~2.1 against
-//     ~2.35 GHz), which slows the kernels around it; in the decoder (K
-//     2048 and 8192) it still gains end to end: QKV and paired gate/up 2 %
-//     (5.00 vs 5.09 ms), the output and down projections another 2.5 %
-//     (4.82 vs 4.95 ms).  MK_GEMM_PIPE_K moves the threshold, MK_GEMM_PIPE=0
-//     keeps the ring kernel.
-//   - K <= 256 with fewer 256 x 256 tiles than CUs: the 128 x 128 kernel
-//     with all of K in LDS: 2048^2 x 256 7.9 against 12.1 (128-tile
-//     kernel); 1024^2 x 256 5.7 / 10.5; 4 x 1024^2 x 128 6.1 / 9.1 (9.9
-//     persistent).
-//   - K <= 128 with a tile per CU or more: the persistent kernel (the next
-//     tile's loads under the current tile's stores): 16 x 2048^2 x 128 48.5
-//     against 54.2 (ring) / 58.6 (128 x 128 all-K-in-LDS).
-//     MK_GEMM_PERSIST=0 turns it off.
-//   - MK_GEMM_SHORTK sets the largest K of the 128 x 128 all-K-in-LDS
-//     kernel (default 256 on 256-multiples, 128 on other 128-multiples;
-//     0: never).
-int default_route(int64_t batch, int64_t M, int64_t N, int64_t K, int epi, int out_f32) {
-  const char* dma_env = getenv("MK_GEMM_DMA");
-  const bool dma = !(dma_env && dma_env[0] == '0');
-  const bool simple_epi = epi == MK_EPI_NONE || epi == MK_EPI_ADD || epi == MK_EPI_SWIGLU;
+//   - K <= 128 with a 256 x 256 tile per CU or more: the persistent kernel
+//     (the next tile's loads under the current tile's stores): 16 x 2048^2 x
+//     128 48.5 against 54.2 (ring).  MK_GEMM_PERSIST=0 turns it off.
+//   - K <= 256 on 128-multiples, fewer 256 x 256 tiles than CUs: the 128 x
+//     128 kernel with all of K in LDS.  MK_GEMM_SHORTK sets its largest K
+//     (default 256 on 256-multiples, 128 on other 128-multiples; 0: never).
+//   - else the tile shape whose estimated time is least (gemm_tile.hip).
+//     The pipelined 256 x 256 kernel stands in for the family's 256 x 256
+//     tiles where M and N divide, 6 % faster there (4096^3 112.7 against
+//     119.1; 128 x 128 tiles 136, hipBLASLt 110).  The estimate moves the
+//     products that do not fill 256 CUs with such tiles to smaller ones:
+//     2048^3 24.8 (128 x 128) against 45 (pipelined), 1024^3 7.9 (64 x 64)
+//     against 25, 256 x 4096 x 4096 20.3 (64 x 64) against 79.
+int default_route(const mkg::TileGemm& g) {
+  const int64_t batch = g.batch, M = g.M, N = g.N, K = g.K;
+  const int epi = g.epi, out_f32 = g.out_f32 ? 1 : 0;
   const int64_t big_tiles = ((M + 255) / 256) * ((N + 255) / 256) * batch;
   const int env_t = env_tile();
-  int tile = env_t;
-  if (tile == 0) tile = big_tiles >= 128 ? 256 : 128;
-  if (epi == MK_EPI_SWIGLU_PAIRS) tile = 256;
   const bool a256 = M % 256 == 0 && N % 256 == 0 && K % 32 == 0;
-  const char* sk = getenv("MK_GEMM_SHORTK");
-  const int64_t shortk_max = std::min<int64_t>(sk ? atoll(sk) : (a256 ? 256 : 128), 256);
-  const char* pe = getenv("MK_GEMM_PERSIST");
-  const bool persist_on = !(pe && pe[0] == '0') && dma;
-  const int cus = device_cus();
-  if (a256 && env_t == 0 && persist_on && big_tiles >= cus && route_fits(MK_GEMM_ROUTE_PERSIST, M, N, K, epi, out_f32))
-    return MK_GEMM_ROUTE_PERSIST;
-  if (K <= shortk_max && (!a256 || big_tiles < cus || !persist_on) && env_t == 0 &&
-      route_fits(MK_GEMM_ROUTE_SHORT, M, N, K, epi, out_f32))
-    return MK_GEMM_ROUTE_SHORT;
   const char* pv = getenv("MK_GEMM_PIPE");
   const char* pk = getenv("MK_GEMM_PIPE_K");
   const int64_t pipe_k = pk ? atoll(pk) : 512;
   const bool pipe = !(pv && atoi(pv) == 0) && K >= pipe_k && route_fits(MK_GEMM_ROUTE_PIPE, M, N, K, epi, out_f32);
-  if (dma && a256 && (tile == 256 || (pipe && env_t == 0)))
-    return pipe ? MK_GEMM_ROUTE_PIPE : MK_GEMM_ROUTE_RING;
-  if (!simple_epi) return MK_GEMM_ROUTE_RING;  // paired SwiGLU: checked aligned by the caller
-  if (tile == 256 && route_fits(MK_GEMM_ROUTE_REG256, M, N, K, epi, out_f32)) return MK_GEMM_ROUTE_REG256;
-  return tile == 256 ? MK_GEMM_ROUTE_GENERIC256 : MK_GEMM_ROUTE_GENERIC128;
+  const int big = pipe ? MK_GEMM_ROUTE_PIPE : MK_GEMM_ROUTE_RING;
+  if (epi == MK_EPI_SWIGLU_PAIRS) return big;  // checked aligned by the caller
+  if (env_t == 128) return MK_GEMM_ROUTE_T128x128;
+  if (!g.registers) {
+    if (env_t == 256) return a256 ? big : MK_GEMM_ROUTE_T256x256;
+    const char* sk = getenv("MK_GEMM_SHORTK");
+    const int64_t shortk_max = std::min<int64_t>(sk ? atoll(sk) : (a256 ? 256 : 128), 256);
+    const char* pe = getenv("MK_GEMM_PERSIST");
+    const bool persist_on = !(pe && pe[0] == '0');
+    const int cus = device_cus();
+    if (a256 && persist_on && big_tiles >= cus && route_fits(MK_GEMM_ROUTE_PERSIST, M, N, K, epi, out_f32))
+      return MK_GEMM_ROUTE_PERSIST;
+    if (K <= shortk_max && (!a256 || big_tiles < cus || !persist_on) &&
+        route_fits(MK_GEMM_ROUTE_SHORT, M, N, K, epi, out_f32))
+      return MK_GEMM_ROUTE_SHORT;
+  }
+  const int s = mkg::tile_pick(g);
+  if (a256 && !g.registers &&
+      (s == mkg::T256x256 || 0.94 * mkg::tile_estimate(g, mkg::T256x256) <= mkg::tile_estimate(g, s)))
+    return big;
+  return MK_GEMM_ROUTE_T16x64 + s;
 }
 
 hipError_t launch_route(int route, const mk::GemmArgs& p, int64_t batch, hipStream_t st) {
@@ -1383,24 +1087,15 @@ hipError_t launch_route(int route, const mk::GemmArgs& p, int64_t batch, hipStre
       }
       break;
     }
-    case MK_GEMM_ROUTE_REG256: {
-      constexpr size_t lds = (size_t)2 * (256 * 64 + 64 * 256) * 2;
-      const dim3 grid((unsigned)((M / 256) * (N / 256)), 1, (unsigned)batch);
-      if (four_waves) {
-        e = lds_opt_in((const void*)mk::gemm_bf16_256_kernel<2, 2>, lds);
-        if (e == hipSuccess) hipLaunchKernelGGL((mk::gemm_bf16_256_kernel<2, 2>), grid, dim3(256), lds, st, p);
-      } else {
-        e = lds_opt_in((const void*)mk::gemm_bf16_256_kernel<2, 4>, lds);
-        if (e == hipSuccess) hipLaunchKernelGGL((mk::gemm_bf16_256_kernel<2, 4>), grid, dim3(512), lds, st, p);
-      }
-      break;
-    }
+    // The names of kernels the tile family replaced.
+    case MK_GEMM_ROUTE_REG256:
     case MK_GEMM_ROUTE_GENERIC256:
-      return launch_bf16<256, 256, 2, 2>(p, (int)batch, st);
+      return mkg::tile_launch(tile_args(p, batch), mkg::T256x256, st);
     case MK_GEMM_ROUTE_GENERIC128:
-      return launch_bf16<128, 128, 2, 2>(p, (int)batch, st);
+      return mkg::tile_launch(tile_args(p, batch), mkg::T128x128, st);
     default:
-      return hipErrorInvalidValue;
+      if (route < MK_GEMM_ROUTE_T16x64 || route > MK_GEMM_ROUTE_T256x256) return hipErrorInvalidValue;
+      return mkg::tile_launch(tile_args(p, batch), route - MK_GEMM_ROUTE_T16x64, st);
   }
   if (e == hipSuccess) e = hipGetLastError();
   return e;
@@ -1433,7 +1128,13 @@ int run_gemm_bf16(const char* fn, const void* a, const void* b, void* c, const v
   p.aux = static_cast<const uint16_t*>(aux);
   hipStream_t st = static_cast<hipStream_t>(stream);
   hipError_t e;
-  if (bt) {
+  const mkg::TileGemm tg = tile_args(p, batch, bt);
+  // B^T: the smaller tiles where the estimate prefers them, as for [K, N].
+  const int bt_shape = bt && epi != MK_EPI_SWIGLU_PAIRS && !tg.registers ? mkg::tile_pick(tg) : mkg::T256x256;
+  if (bt && bt_shape != mkg::T256x256 &&
+      mkg::tile_estimate(tg, bt_shape) < 0.94 * mkg::tile_estimate(tg, mkg::T256x256)) {
+    e = mkg::tile_launch(tg, bt_shape, st);
+  } else if (bt) {
     const dim3 grid((unsigned)((M / 256) * (N / 256)), 1, (unsigned)batch);
     const char* pv = getenv("MK_GEMM_PIPE");
     const char* pk = getenv("MK_GEMM_PIPE_K");
@@ -1452,7 +1153,7 @@ int run_gemm_bf16(const char* fn, const void* a, const void* b, void* c, const v
     }
     if (e == hipSuccess) e = hipGetLastError();
   } else {
-    if (route == MK_GEMM_ROUTE_DEFAULT) route = default_route(batch, M, N, K, epi, out_f32);
+    if (route == MK_GEMM_ROUTE_DEFAULT) route = default_route(tg);
     else if (!route_fits(route, M, N, K, epi, out_f32))
       return mkc::fail(MK_EUNSUPPORTED, "%s: route %d does not take this product (M=%lld, N=%lld, K=%lld, "
                        "epilogue %d, f32 output %d)", fn, route, (long long)M, (long long)N, (long long)K, epi,
@@ -1484,7 +1185,7 @@ extern "C" int mk_gemm_bf16_nt(const void* a, const void* bt, void* c, const voi
 extern "C" int mk_gemm_bf16_route(const void* a, const void* b, void* c, const void* aux, int epilogue,
                                   int64_t batch, int64_t M, int64_t N, int64_t K, int out_f32, int route,
                                   void* stream) {
-  if (route < MK_GEMM_ROUTE_DEFAULT || route >= MK_GEMM_ROUTE_COUNT)
+  if (route != MK_GEMM_ROUTE_DEFAULT && !route_known(route))
     return mkc::fail(MK_EINVAL, "mk_gemm_bf16_route: unknown route %d", route);
   return run_gemm_bf16("mk_gemm_bf16_route", a, b, c, aux, epilogue, batch, M, N, K, out_f32, stream, false, route);
 }
@@ -1577,6 +1278,7 @@ extern "C" int mk_gemm_bf16_autotune(const void* a, const void* b, void* c, cons
   int rc = MK_OK;
   for (int r = 1; r < MK_GEMM_ROUTE_COUNT && rc == MK_OK; ++r) {
     if (!route_fits(r, M, N, K, epilogue, out_f32)) continue;
+    if (r >= MK_GEMM_ROUTE_REG256 && r <= MK_GEMM_ROUTE_GENERIC128) continue;  // other names of tile shapes
     std::vector<float> t;
     for (int i = 0; i < warm + iters && rc == MK_OK; ++i) {
       if (i >= warm && hipEventRecord(ev[0], st) != hipSuccess) rc = mkc::fail(MK_ELAUNCH, "%s: event record", fn);
@@ -1673,7 +1375,7 @@ extern "C" int mk_gemm_autotune_load(const char* path) {
     if (line[0] == '\n') continue;
     if (sscanf(line, "%63s %d %lld %lld %lld %lld %d %d %d %f %c", arch, &cus, &b, &m, &n, &k, &ecls, &of, &route,
                &us, &extra) != 10 || cus <= 0 || b <= 0 || m <= 0 || n <= 0 || k <= 0 || ecls < 0 || ecls > 2 ||
-        (of != 0 && of != 1) || route <= MK_GEMM_ROUTE_DEFAULT || route >= MK_GEMM_ROUTE_COUNT || !(us >= 0.f)) {
+        (of != 0 && of != 1) || !route_known(route) || !(us >= 0.f)) {
       fclose(f);
       return -mkc::fail(MK_EINVAL, "mk_gemm_autotune_load: %s line %d is malformed", path, lineno);
     }

@@ -18,7 +18,8 @@ MK_DT_F32, MK_DT_BF16 = 0, 1
 MK_EPI_NONE, MK_EPI_ADD, MK_EPI_SWIGLU, MK_EPI_SWIGLU_PAIRS = 0, 1, 2, 3
 # bf16 GEMM routes (MK_GEMM_ROUTE_*)
 GEMM_ROUTES = {"default": 0, "ring": 1, "pipe": 2, "persist": 3, "short": 4, "reg256": 5, "generic256": 6,
-               "generic128": 7}
+               "generic128": 7, "t16x64": 16, "t32x64": 17, "t64x64": 18, "t128x64": 19, "t128x128": 20,
+               "t256x256": 21}
 MK_REDUCE_SUM, MK_REDUCE_MAX, MK_REDUCE_MIN = 0, 1, 2
 EW_OPS = ["LOAD", "CONST", "ADD", "SUB", "MUL", "DIV", "MAX", "MIN", "POW", "NEG", "ABS", "EXP", "LOG",
           "LOG1P", "EXPM1", "TANH", "RSQRT", "SQRT", "LOGISTIC", "FLOOR", "CEIL", "CMP_EQ", "CMP_NE",
