@@ -11,12 +11,16 @@
 //   * K == 0 is handled by the planner (zeros, :832-845);
 //   * any K and N, and operands read through strides, so a transposed
 //     operand (a @ a.T) or a vector needs no copy.
-// Floating inputs (f32, bf16, f16; both the same type) accumulate in f32 in
-// k order and store f32, bf16 or f16 (round to nearest even).
+// Floating inputs (f32, bf16, f16; both the same type) accumulate in f32
+// and store f32, bf16 or f16 (round to nearest even).
 //
-// One thread per output element, grid-stride: these are the shapes the
-// tiled kernels reject, not throughput paths.
+// bf16 and f16 products of K >= 16 run on the tile family (gemm_tile.hip),
+// which reads either storage order at any row stride in place: a linear
+// layer's gradients (dy W^T, x^T dy), odd sizes, f16.  The rest -- integers,
+// f32, short sums, strides that leave no contiguous dimension -- has one
+// thread per output element, grid-stride.
 #include "common.h"
+#include "gemm_tile.h"
 
 namespace mk {
 
@@ -98,6 +102,48 @@ namespace {
 bool is_int(int t) { return t >= mk::kS8 && t <= mk::kU64; }
 bool is_float(int t) { return t == mk::kF16 || t == mk::kF32 || t == mk::kBF16; }
 
+// One operand's row stride if one of its two dimensions is contiguous and
+// its rows do not overlap: x (m or n, extent X) or k (extent K).
+bool operand_order(int64_t sx, int64_t sk, int64_t X, int64_t K, bool* x_contiguous, int64_t* ld) {
+  if (sk == 1 && (X == 1 || sx >= K)) {
+    *x_contiguous = false;
+    *ld = X == 1 ? K : sx;
+    return true;
+  }
+  if ((X == 1 || sx == 1) && sk >= X) {
+    *x_contiguous = true;
+    *ld = sk;
+    return true;
+  }
+  return false;
+}
+
+// The product as the tile family takes it, if it does.  Short sums stay on
+// the thread-per-output kernel: below 16 most of a 32-k step is padding.
+bool tile_form(const mk::DotArgs& p, int type, mkg::TileGemm* g) {
+  if ((type != mk::kBF16 && type != mk::kF16) || p.K < 16) return false;
+  const int64_t top = (int64_t)1 << 30;
+  if (p.M > top || p.N > top || p.K > top || p.batch > 65535 || ((p.M + 15) / 16) * ((p.N + 63) / 64) > INT32_MAX)
+    return false;
+  bool n_contiguous = false;
+  if (!operand_order(p.sa[1], p.sa[2], p.M, p.K, &g->a_t, &g->lda) ||
+      !operand_order(p.sb[2], p.sb[1], p.N, p.K, &n_contiguous, &g->ldb))
+    return false;
+  g->b_t = !n_contiguous;
+  g->a = p.a;
+  g->b = p.b;
+  g->c = p.c;
+  g->batch = p.batch;
+  g->M = p.M;
+  g->N = p.N;
+  g->K = p.K;
+  g->sa = p.sa[0];
+  g->sb = p.sb[0];
+  g->f16 = type == mk::kF16;
+  g->out_f32 = p.out_type == mk::kF32;
+  return true;
+}
+
 }  // namespace
 
 extern "C" int mk_dot_general(int type_a, int type_b, int type_out, const void* a, const void* b, void* c,
@@ -123,6 +169,12 @@ extern "C" int mk_dot_general(int type_a, int type_b, int type_out, const void* 
   p.batch = batch; p.M = M; p.N = N; p.K = K;
   for (int i = 0; i < 3; ++i) { p.sa[i] = a_strides[i]; p.sb[i] = b_strides[i]; }
   p.out_type = type_out;
+  mkg::TileGemm g;
+  if (tile_form(p, type_a, &g)) {
+    const hipError_t te = mkg::tile_launch(g, mkg::tile_pick(g), static_cast<hipStream_t>(stream));
+    if (te != hipSuccess) return mkc::fail(MK_ELAUNCH, "%s: launch failed: %s", fn, hipGetErrorString(te));
+    return MK_OK;
+  }
   const int64_t total = batch * M * N;
   const unsigned grid = (unsigned)std::min<int64_t>((total + 255) / 256, 65536);
   hipStream_t st = static_cast<hipStream_t>(stream);
