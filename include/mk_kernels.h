@@ -152,7 +152,8 @@ int mk_int4g64_matmul_bf16_noalloc(const void* x, const void* w_packed, const vo
  * mk_gemm_bf16: bf16 inputs, f32 accumulation; C is bf16 (out_f32 = 0) or
  *   f32 (out_f32 = 1, dot_general with preferred_element_type = f32,
  *   binary_ops.mm:775-782).
- * mk_gemm_f32:  f32 inputs and output, f32 products and accumulation.
+ * mk_gemm_f32:  f32 inputs and output, f32 products and accumulation (to
+ *   f32 accuracy on the bf16 matrix cores: gemm_split.hip).
  * Both need K % 8 == 0 and N % 8 == 0 (else MK_EUNSUPPORTED).
  * ---------------------------------------------------------------------- */
 int mk_gemm_bf16(const void* a, const void* b, void* c, int64_t batch, int64_t M, int64_t N,
@@ -285,9 +286,9 @@ const char* mk_gemm_autotune_header(void);
  * b*a_strides[0] + m*a_strides[1] + k*a_strides[2] of a, B[b, k, n] element
  * b*b_strides[0] + k*b_strides[1] + n*b_strides[2] of b; C is contiguous
  * [batch, M, N].  Types use the PJRT_Buffer_Type numbering below; both
- * operands must have the same type (MK_EUNSUPPORTED otherwise).  bf16 and
- * f16 operands with one contiguous dimension each run on the matrix cores
- * from K = 16; the rest has one thread per output element. */
+ * operands must have the same type (MK_EUNSUPPORTED otherwise).  Floating
+ * operands with one contiguous dimension each run on the matrix cores from
+ * K = 16; the rest has one thread per output element. */
 enum {
   MK_TYPE_S8 = 2, MK_TYPE_S16 = 3, MK_TYPE_S32 = 4, MK_TYPE_S64 = 5, MK_TYPE_U8 = 6, MK_TYPE_U16 = 7,
   MK_TYPE_U32 = 8, MK_TYPE_U64 = 9, MK_TYPE_F16 = 10, MK_TYPE_F32 = 11, MK_TYPE_BF16 = 13

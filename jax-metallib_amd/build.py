@@ -43,6 +43,7 @@ KERNEL_SOURCES = [
     "kernels/decoder.hip",
     "kernels/gemm.hip",
     "kernels/gemm_tile.hip",
+    "kernels/gemm_split.hip",
     "kernels/dot_general.hip",
     "kernels/rowops.hip",
     "kernels/eltwise.hip",

@@ -14,12 +14,13 @@
 // Floating inputs (f32, bf16, f16; both the same type) accumulate in f32
 // and store f32, bf16 or f16 (round to nearest even).
 //
-// bf16 and f16 products of K >= 16 run on the tile family (gemm_tile.hip),
-// which reads either storage order at any row stride in place: a linear
-// layer's gradients (dy W^T, x^T dy), odd sizes, f16.  The rest -- integers,
-// f32, short sums, strides that leave no contiguous dimension -- has one
-// thread per output element, grid-stride.
+// Floating products of K >= 16 run on the tiled kernels (gemm_tile.hip: bf16
+// and f16; gemm_split.hip: f32), which read either storage order at any row
+// stride in place: a linear layer's gradients (dy W^T, x^T dy), odd sizes.
+// The rest -- integers, short sums, strides that leave no contiguous
+// dimension -- has one thread per output element, grid-stride.
 #include "common.h"
+#include "gemm_split.h"
 #include "gemm_tile.h"
 
 namespace mk {
@@ -118,10 +119,11 @@ bool operand_order(int64_t sx, int64_t sk, int64_t X, int64_t K, bool* x_contigu
   return false;
 }
 
-// The product as the tile family takes it, if it does.  Short sums stay on
-// the thread-per-output kernel: below 16 most of a 32-k step is padding.
-bool tile_form(const mk::DotArgs& p, int type, mkg::TileGemm* g) {
-  if ((type != mk::kBF16 && type != mk::kF16) || p.K < 16) return false;
+// How the tiled kernels read the product's operands, if they do.  Short sums
+// stay on the thread-per-output kernel: below 16 most of a 32-k step is
+// padding.
+bool tile_form(const mk::DotArgs& p, mkg::TileGemm* g) {
+  if (p.K < 16) return false;
   const int64_t top = (int64_t)1 << 30;
   if (p.M > top || p.N > top || p.K > top || p.batch > 65535 || ((p.M + 15) / 16) * ((p.N + 63) / 64) > INT32_MAX)
     return false;
@@ -139,9 +141,30 @@ bool tile_form(const mk::DotArgs& p, int type, mkg::TileGemm* g) {
   g->K = p.K;
   g->sa = p.sa[0];
   g->sb = p.sb[0];
-  g->f16 = type == mk::kF16;
-  g->out_f32 = p.out_type == mk::kF32;
   return true;
+}
+
+hipError_t launch_tiled(mkg::TileGemm g, int type, int out_type, hipStream_t st) {
+  if (type == mk::kF32) {
+    mkg::SplitGemm s;
+    s.a = static_cast<const float*>(g.a);
+    s.b = static_cast<const float*>(g.b);
+    s.c = static_cast<float*>(g.c);
+    s.batch = g.batch;
+    s.M = g.M;
+    s.N = g.N;
+    s.K = g.K;
+    s.lda = g.lda;
+    s.ldb = g.ldb;
+    s.sa = g.sa;
+    s.sb = g.sb;
+    s.a_t = g.a_t;
+    s.b_t = g.b_t;
+    return mkg::split_launch(s, 0, st);
+  }
+  g.f16 = type == mk::kF16;
+  g.out_f32 = out_type == mk::kF32;
+  return mkg::tile_launch(g, mkg::tile_pick(g), st);
 }
 
 }  // namespace
@@ -170,8 +193,8 @@ extern "C" int mk_dot_general(int type_a, int type_b, int type_out, const void* 
   for (int i = 0; i < 3; ++i) { p.sa[i] = a_strides[i]; p.sb[i] = b_strides[i]; }
   p.out_type = type_out;
   mkg::TileGemm g;
-  if (tile_form(p, type_a, &g)) {
-    const hipError_t te = mkg::tile_launch(g, mkg::tile_pick(g), static_cast<hipStream_t>(stream));
+  if (floats && tile_form(p, &g)) {
+    const hipError_t te = launch_tiled(g, type_a, type_out, static_cast<hipStream_t>(stream));
     if (te != hipSuccess) return mkc::fail(MK_ELAUNCH, "%s: launch failed: %s", fn, hipGetErrorString(te));
     return MK_OK;
   }

@@ -5,7 +5,7 @@
 //
 // bf16 x bf16 -> f32 accumulation -> bf16 or f32 output
 //   (preferred_element_type = f32 returns f32, binary_ops.mm:775-782)
-// f32  x f32  -> f32 (v_mfma_f32_16x16x4_f32, full f32 products)
+// f32  x f32  -> f32 (gemm_split.hip)
 //
 // The bf16 kernels here take M and N in multiples of 256 (128 for the
 // short-K one); gemm_tile.hip takes every other shape, and these where its
@@ -16,6 +16,7 @@
 // the A panels and B panels they share stay in that XCD's L2.
 #include "common.h"
 #include "epilogue.h"
+#include "gemm_split.h"
 #include "gemm_tile.h"
 
 namespace mk {
@@ -45,146 +46,6 @@ __device__ __forceinline__ void tile_coords(uint32_t L, int tiles_m, int tiles_n
     tn = (int)L - tm * tiles_n;
   }
 }
-
-// f32 GEMM: v_mfma_f32_16x16x4_f32.  Within each 32-k chunk a lane of k
-// block j (= lane / 16) feeds k = 8j + s to the s-th MFMA, for both operands,
-// so a fragment is 8 consecutive floats of one row (two 16-byte LDS reads).
-template <int BM, int BN, int WM, int WN>
-__global__ __launch_bounds__(WM * WN * 64) void gemm_f32_kernel(GemmArgs p) {
-  constexpr int BK = 32;
-  constexpr int LDK = BK + 4;  // padded row length (floats): 144 B
-  constexpr int NT = WM * WN * 64;
-  constexpr int TM = BM / WM / 16;
-  constexpr int TN = BN / WN / 16;
-  constexpr int ACH = BM * BK / 4 / NT;          // A 16-byte chunks per thread
-  constexpr int BTOT = (BK / 4) * (BN / 4);      // B 4x4 blocks per tile
-  constexpr int BBL = (BTOT + NT - 1) / NT;      // B blocks per thread
-  static_assert(ACH * NT * 4 == BM * BK, "A staging must divide evenly");
-
-  extern __shared__ __align__(16) unsigned char smem[];
-  float* As = reinterpret_cast<float*>(smem);  // [2][BM][LDK]
-  float* Bs = As + 2 * BM * LDK;               // [2][BN][LDK]
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave / WN, wn = wave % WN;
-  const int tiles_m = (p.M + BM - 1) / BM, tiles_n = (p.N + BN - 1) / BN;
-  int tm, tn;
-  tile_coords(xcd_logical_id(blockIdx.x, gridDim.x), tiles_m, tiles_n, tm, tn);
-  const int m0 = tm * BM, n0 = tn * BN;
-  const float* A = static_cast<const float*>(p.a) + (size_t)blockIdx.z * p.sa;
-  const float* B = static_cast<const float*>(p.b) + (size_t)blockIdx.z * p.sb;
-  const int M = p.M, N = p.N, K = p.K;
-
-  f32x4 ra[ACH];
-  f32x4 rb[BBL][4];
-
-  auto load_tile = [&](int k0) {
-#pragma unroll
-    for (int i = 0; i < ACH; ++i) {
-      const int q = tid + i * NT;
-      const int row = q / (BK / 4), kc = q % (BK / 4);
-      const int gm = m0 + row, gk = k0 + 4 * kc;
-      ra[i] = (gm < M && gk < K) ? *reinterpret_cast<const f32x4*>(A + (size_t)gm * K + gk)
-                                 : f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-#pragma unroll
-    for (int i = 0; i < BBL; ++i) {
-      const int q = tid + i * NT;
-      const int kb = q / (BN / 4), nb = q % (BN / 4);
-      const int gn = n0 + 4 * nb;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int gk = k0 + 4 * kb + r;
-        rb[i][r] = (q < BTOT && gn < N && gk < K) ? *reinterpret_cast<const f32x4*>(B + (size_t)gk * N + gn)
-                                      : f32x4{0.f, 0.f, 0.f, 0.f};
-      }
-    }
-  };
-
-  auto store_tile = [&](int buf) {
-    float* as = As + buf * BM * LDK;
-    float* bs = Bs + buf * BN * LDK;
-#pragma unroll
-    for (int i = 0; i < ACH; ++i) {
-      const int q = tid + i * NT;
-      const int row = q / (BK / 4), kc = q % (BK / 4);
-      *reinterpret_cast<f32x4*>(as + row * LDK + 4 * kc) = ra[i];
-    }
-#pragma unroll
-    for (int i = 0; i < BBL; ++i) {
-      const int q = tid + i * NT;
-      if (q >= BTOT) break;
-      const int kb = q / (BN / 4), nb = q % (BN / 4);
-      *reinterpret_cast<f32x4*>(bs + (4 * nb + 0) * LDK + 4 * kb) =
-          f32x4{rb[i][0].x, rb[i][1].x, rb[i][2].x, rb[i][3].x};
-      *reinterpret_cast<f32x4*>(bs + (4 * nb + 1) * LDK + 4 * kb) =
-          f32x4{rb[i][0].y, rb[i][1].y, rb[i][2].y, rb[i][3].y};
-      *reinterpret_cast<f32x4*>(bs + (4 * nb + 2) * LDK + 4 * kb) =
-          f32x4{rb[i][0].z, rb[i][1].z, rb[i][2].z, rb[i][3].z};
-      *reinterpret_cast<f32x4*>(bs + (4 * nb + 3) * LDK + 4 * kb) =
-          f32x4{rb[i][0].w, rb[i][1].w, rb[i][2].w, rb[i][3].w};
-    }
-  };
-
-  f32x4 acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  const int KT = (K + BK - 1) / BK;
-  load_tile(0);
-  store_tile(0);
-  __syncthreads();
-
-  const int arow = wm * TM * 16 + (lane & 15);
-  const int brow = wn * TN * 16 + (lane & 15);
-  const int kofs = 8 * (lane >> 4);
-
-  for (int kt = 0; kt < KT; ++kt) {
-    const int buf = kt & 1;
-    if (kt + 1 < KT) load_tile((kt + 1) * BK);
-    const float* as = As + buf * BM * LDK;
-    const float* bs = Bs + buf * BN * LDK;
-    f32x4 af[TM][2], bf[TN][2];
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      af[i][0] = *reinterpret_cast<const f32x4*>(as + (arow + 16 * i) * LDK + kofs);
-      af[i][1] = *reinterpret_cast<const f32x4*>(as + (arow + 16 * i) * LDK + kofs + 4);
-    }
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      bf[j][0] = *reinterpret_cast<const f32x4*>(bs + (brow + 16 * j) * LDK + kofs);
-      bf[j][1] = *reinterpret_cast<const f32x4*>(bs + (brow + 16 * j) * LDK + kofs + 4);
-    }
-#pragma unroll
-    for (int s = 0; s < 8; ++s) {
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bf[j][s >> 2][s & 3], af[i][s >> 2][s & 3],
-                                                          acc[i][j], 0, 0, 0);
-    }
-    if (kt + 1 < KT) store_tile(buf ^ 1);
-    __syncthreads();
-  }
-
-  float* C = static_cast<float*>(p.c) + (size_t)blockIdx.z * p.sc;
-  const int mrow = m0 + wm * TM * 16 + (lane & 15);
-  const int ncol = n0 + wn * TN * 16 + 4 * (lane >> 4);
-#pragma unroll
-  for (int i = 0; i < TM; ++i) {
-    const int m = mrow + 16 * i;
-    if (m >= M) continue;
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int n = ncol + 16 * j;
-      if (n < N) *reinterpret_cast<f32x4*>(C + (size_t)m * N + n) = acc[i][j];
-    }
-  }
-}
-
 
 // gfx950's transposing LDS read, ds_read_b64_tr_b16: within each 16-lane
 // group, lanes 4r + q name the 8 bytes of row r, columns 4q..4q+3 of a
@@ -870,18 +731,6 @@ hipError_t lds_opt_in(const void* fn, size_t bytes) {
   return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
 }
 
-template <int BM, int BN, int WM, int WN>
-hipError_t launch_f32(const mk::GemmArgs& a, int batch, hipStream_t st) {
-  constexpr size_t lds = (size_t)2 * (BM + BN) * (32 + 4) * 4;
-  const void* fn = (const void*)mk::gemm_f32_kernel<BM, BN, WM, WN>;
-  hipError_t e = lds_opt_in(fn, lds);
-  if (e != hipSuccess) return e;
-  const int tiles = ((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN);
-  hipLaunchKernelGGL((mk::gemm_f32_kernel<BM, BN, WM, WN>), dim3(tiles, 1, batch),
-                     dim3(WM * WN * 64), lds, st, a);
-  return hipGetLastError();
-}
-
 int check_gemm(const char* fn, const void* a, const void* b, void* c, int64_t batch, int64_t M,
                int64_t N, int64_t K) {
   if (!a || !b || !c) return mkc::fail(MK_EINVAL, "%s: null pointer argument", fn);
@@ -1400,22 +1249,21 @@ extern "C" int mk_gemm_f32(const void* a, const void* b, void* c, int64_t batch,
   mkc::clear_error();
   int rc = check_gemm("mk_gemm_f32", a, b, c, batch, M, N, K);
   if (rc != MK_OK) return rc;
-  mk::GemmArgs p;
-  p.a = a; p.b = b; p.c = c;
-  p.M = (int)M; p.N = (int)N; p.K = (int)K;
-  p.sa = M * K; p.sb = K * N; p.sc = M * N;
-  p.out_f32 = 1;
-  p.epi = MK_EPI_NONE;
-  p.aux = nullptr;
-  // 128 x 128 tiles once they fill the chip (2048^3: 170 us against 183 us
-  // with 64 x 64); below about 192 of them 64 x 64 tiles, four times as many
-  // workgroups (1024^3: 35 us against 86 us).  Same k order, same bits.
-  // MK_GEMM_F32_TILE=64 / 128 overrides.
-  const int64_t t128 = ((M + 127) / 128) * ((N + 127) / 128) * batch;
+  mkg::SplitGemm g;
+  g.a = static_cast<const float*>(a);
+  g.b = static_cast<const float*>(b);
+  g.c = static_cast<float*>(c);
+  g.batch = batch;
+  g.M = M;
+  g.N = N;
+  g.K = K;
+  g.lda = K;
+  g.ldb = N;
+  g.sa = M * K;
+  g.sb = K * N;
+  // MK_GEMM_F32_TILE=16 / 64 / 128 overrides the tile: the same bits.
   const char* ft = getenv("MK_GEMM_F32_TILE");
-  const int tile = ft ? atoi(ft) : (t128 < 192 ? 64 : 128);
-  hipError_t e = tile == 64 ? launch_f32<64, 64, 2, 2>(p, (int)batch, static_cast<hipStream_t>(stream))
-                            : launch_f32<128, 128, 2, 2>(p, (int)batch, static_cast<hipStream_t>(stream));
+  const hipError_t e = mkg::split_launch(g, ft ? atoi(ft) : 0, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return mkc::fail(MK_ELAUNCH, "mk_gemm_f32: launch failed: %s", hipGetErrorString(e));
   return MK_OK;
 }

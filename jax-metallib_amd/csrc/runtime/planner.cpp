@@ -1093,14 +1093,15 @@ class Planner {
     }
     const bool fast = !(general && gd.transposed) && dot_shape(op, &d) && fast_types && d.K > 0 &&
                       d.K % 8 == 0 && d.N % 8 == 0 && numel(v) == d.batch * d.M * d.N;
-    // A bf16 lhs stored [K, M] (a weight gradient x^T dy) is read in place by
-    // the general kernel's tiles; so is an rhs stored [N, K] from 2^27
-    // multiply-adds where the GEMM below would copy it (smaller products
-    // keep the copy and the measured route).
+    // An lhs stored [K, M] (a weight gradient x^T dy) is read in place by the
+    // tiled kernels behind mk_dot_general; so is an rhs stored [N, K] from
+    // 2^27 multiply-adds where the GEMM below would copy it (smaller products
+    // keep the copy).
     const bool in_place =
-        general && ta == DT_BF16 && !gd.copy_a && !gd.copy_b && gd.K >= 16 && gd.batch <= 65535 &&
+        general && !gd.copy_a && !gd.copy_b && gd.K >= 16 && gd.batch <= 65535 &&
         ((gd.sa[1] == 1 && gd.sa[2] >= gd.M && gd.M > 1) ||
-         (gd.sb[1] == 1 && gd.sb[2] >= gd.K && (gd.M % 256 != 0 || gd.N % 256 != 0 || gd.K % 32 != 0) &&
+         (gd.sb[1] == 1 && gd.sb[2] >= gd.K &&
+          (ta == DT_F32 || gd.M % 256 != 0 || gd.N % 256 != 0 || gd.K % 32 != 0) &&
           (double)gd.M * (double)gd.N * (double)gd.K >= (double)(int64_t(1) << 27)));
     if (!fast && !in_place && general && fast_types && gd.K > 0 && gd.K % 8 == 0 && gd.N % 8 == 0 &&
         numel(v) == gd.batch * gd.M * gd.N && gd.M * gd.N * gd.K >= (int64_t(1) << 18)) {
