@@ -16,14 +16,15 @@
 //   sum      f32 accumulation, output in the input dtype.
 //   max      NaN-propagating, -0 < +0 (metal_kernels.mm:830-857 order key).
 //
-// Layout: X [rows, cols] row-major.  One 256-thread workgroup per row; each
-// thread caches its share of the row in registers (VPT 16-byte vectors), so
-// the row is read from HBM exactly once and written at most once.  Wave
-// reductions use cross-lane shuffles, then one LDS exchange across the 4
-// waves.  Rows longer than the register cache (or not a multiple of the
-// vector width) take the streaming variant that re-reads the row.  argmax,
-// max and min of rows up to 16 vectors per lane of one wave (32 for bf16)
-// run one wave per row instead (row_wave_kernel).
+// Layout: X [rows, cols] row-major.  One workgroup of 256 or 1024 threads
+// per row; each thread caches its share of the row in registers (VPT 16-byte
+// vectors), so the row is read from HBM exactly once and written at most
+// once.  Wave reductions use cross-lane shuffles, then one LDS exchange
+// across the waves.  Rows that are not 16-byte aligned are read and written
+// with unaligned vectors, the last of a row element by element.  Rows longer
+// than the register cache take the streaming variant that re-reads the row.
+// argmax, max and min of aligned rows up to 16 vectors per lane of one wave
+// (32 for bf16) run one wave per row instead (row_wave_kernel).
 #include "common.h"
 
 #include <math.h>
@@ -34,6 +35,7 @@
 namespace mk {
 
 constexpr int kRowThreads = 256;
+constexpr int kRowMaxThreads = 1024;
 
 // ROW_MIN is max of the negated row, negated back: negation is exact, NaN
 // still propagates and -0 < +0 holds.
@@ -123,35 +125,56 @@ struct Vec<uint16_t> {
   static constexpr bool bf16 = true;
 };
 
-// Workgroup-wide reductions through one LDS exchange (4 waves).
+// Reductions over the NW waves of a row, through one LDS exchange (none for
+// one wave).  With 16 waves each combines the partials by another shuffle.
+template <int NW>
 __device__ __forceinline__ float block_sum(float v, float* red) {
   v = wave_sum(v);
+  if constexpr (NW == 1) return v;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   __syncthreads();
   if (lane == 0) red[wv] = v;
   __syncthreads();
-  return red[0] + red[1] + red[2] + red[3];
+  if constexpr (NW == 4) return red[0] + red[1] + red[2] + red[3];
+  v = red[lane & (NW - 1)];
+#pragma unroll
+  for (int o = NW / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  return v;
 }
 
+template <int NW>
 __device__ __forceinline__ float block_max(float v, float* red) {
   v = wave_max(v);
+  if constexpr (NW == 1) return v;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   __syncthreads();
   if (lane == 0) red[wv] = v;
   __syncthreads();
-  return xmax(xmax(red[0], red[1]), xmax(red[2], red[3]));
+  if constexpr (NW == 4) return xmax(xmax(red[0], red[1]), xmax(red[2], red[3]));
+  v = red[lane & (NW - 1)];
+#pragma unroll
+  for (int o = NW / 2; o > 0; o >>= 1) v = xmax(v, __shfl_xor(v, o, 64));
+  return v;
 }
 
+template <int NW>
 __device__ __forceinline__ int block_min_int(int v, int* red) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o, 64));
+  if constexpr (NW == 1) return v;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   __syncthreads();
   if (lane == 0) red[wv] = v;
   __syncthreads();
-  return min(min(red[0], red[1]), min(red[2], red[3]));
+  if constexpr (NW == 4) return min(min(red[0], red[1]), min(red[2], red[3]));
+  v = red[lane & (NW - 1)];
+#pragma unroll
+  for (int o = NW / 2; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o, 64));
+  return v;
 }
 
+// The first NaN, else the first of the largest, of every thread's (v, i).
+template <int NW>
 __device__ __forceinline__ void block_argmax(float& v, int& i, float* redv, int* redi) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
@@ -168,8 +191,7 @@ __device__ __forceinline__ void block_argmax(float& v, int& i, float* redv, int*
   __syncthreads();
   v = redv[0];
   i = redi[0];
-#pragma unroll
-  for (int w = 1; w < 4; ++w) arg_combine(v, i, redv[w], redi[w]);
+  for (int w = 1; w < NW; ++w) arg_combine(v, i, redv[w], redi[w]);
 }
 
 // Element e of a 16-byte vector of a row, as f32.
@@ -275,38 +297,96 @@ __global__ __launch_bounds__(kRowThreads) void row_wave_kernel(RowArgs a) {
   }
 }
 
-// Register-cached row kernel: the row is covered by 256 threads x VPT vectors
-// (VPT * 256 * Vec::N >= cols, cols % Vec::N == 0, rows 16-byte aligned).
-template <typename T, int OP, int VPT, bool GE = sizeof(T) == 4>
-__global__ __launch_bounds__(kRowThreads) void row_cached_kernel(RowArgs a) {
+typedef u32x4 __attribute__((aligned(2))) u32x4_row;  // a vector of a row at any element
+
+// Vector c of a row of any alignment: its elements past the row's end read
+// as `fill` (f32).
+template <typename T>
+__device__ __forceinline__ void load_any(const T* row, int c, int cols, float fill, float (&o)[Vec<T>::N]) {
+  constexpr int E = Vec<T>::N;
+  if (c + E <= cols) {
+    const u32x4 w = *reinterpret_cast<const u32x4_row*>(row + c);
+#pragma unroll
+    for (int e = 0; e < E; ++e) o[e] = row_elem<T>(w, e);
+  } else {
+#pragma unroll
+    for (int e = 0; e < E; ++e) o[e] = c + e < cols ? Vec<T>::load1(row, c + e) : fill;
+  }
+}
+
+template <typename T>
+__device__ __forceinline__ void store_any(T* row, int c, int cols, const float (&v)[Vec<T>::N]) {
+  constexpr int E = Vec<T>::N;
+  if (c + E <= cols) {
+    u32x4 w;
+    if constexpr (Vec<T>::bf16) w = u32x4{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]),
+                                          pack_bf16x2(v[6], v[7])};
+    else w = u32x4{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])};
+    *reinterpret_cast<u32x4_row*>(row + c) = w;
+  } else {
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+      if (c + e < cols) Vec<T>::store1(row, c + e, v[e]);
+  }
+}
+
+// Register-cached row kernel: the row is covered by NT threads x VPT vectors
+// (VPT * NT * Vec::N >= cols).  ALN: cols % Vec::N == 0 and rows 16-byte
+// aligned; otherwise elements past the row's end are held as the operation's
+// neutral value.
+//
+// NT 64: four rows to a workgroup of 256, one wave each, no barriers (short
+// rows: with 256 threads a row most of them idle, and its barriers cost more
+// than its work).
+//
+// It is bound by memory where rows are many; where they are few, by how
+// much of a row one CU has in flight and by the reductions' latency, which
+// is what 1024 threads are for.  Against 256 threads, or for unaligned and
+// longer rows the scalar streaming kernel (us): 64 x 32001 f32 softmax 46.7 ->
+// 7.0, argmax 22.4 -> 4.6; 4096 x 5001 bf16 softmax 47.0 -> 18.5; 2048 x
+// 20000 f32 softmax 119.7 -> 56.1; 64 x 32000 bf16 RMSNorm 8.5 -> 4.7.
+template <typename T, int OP, int VPT, int NT, bool ALN, bool GE = sizeof(T) == 4>
+__global__ __launch_bounds__(NT < kRowThreads ? kRowThreads : NT) void row_cached_kernel(RowArgs a) {
   using V = Vec<T>;
-  constexpr int E = V::N;
-  __shared__ float redf[4];
-  __shared__ int redi[4];
+  constexpr int E = V::N, NW = NT / kWave, RPB = NT < kRowThreads ? kRowThreads / NT : 1;
+  constexpr float kFill = OP == ROW_RMSNORM || OP == ROW_SUM ? 0.f : OP == ROW_MIN ? INFINITY : -INFINITY;
+  __shared__ float redf[NW];
+  __shared__ int redi[NW];
+  const int tid = RPB > 1 ? threadIdx.x % NT : threadIdx.x;
+  const int sub = RPB > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / NT) : 0;
+  const int cols = (int)a.cols;  // at most 65536 here
   // Rows are strided over the grid (the launch caps it), so any row count
-  // fits a launch; every wave of a workgroup runs the same iterations, so
-  // the barriers inside the reductions stay uniform.
-  for (int64_t row = blockIdx.x; row < a.rows; row += gridDim.x) {
-  const int64_t base = row * a.cols;
-  const int tid = threadIdx.x;
+  // fits a launch; every wave of a row runs the same iterations, so the
+  // barriers inside the reductions stay uniform.
+  for (int64_t row = (int64_t)blockIdx.x * RPB + sub; row < a.rows; row += (int64_t)gridDim.x * RPB) {
+  const T* xr = static_cast<const T*>(a.x) + row * a.cols;
+  T* yr = static_cast<T*>(a.y) + row * a.cols;  // softmax, RMSNorm
   float v[VPT][E];
   bool ok[VPT];
 #pragma unroll
   for (int q = 0; q < VPT; ++q) {
-    const int64_t c = (int64_t)(q * kRowThreads + tid) * E;
-    ok[q] = c < a.cols;
-    if (ok[q]) V::load(a.x, base + c, v[q]);
+    const int c = (q * NT + tid) * E;
+    ok[q] = c < cols;
+    if (ok[q]) {
+      if constexpr (ALN) V::load(xr, c, v[q]);
+      else load_any<T>(xr, c, cols, kFill, v[q]);
+    }
   }
+  auto store = [&](int q) {
+    const int c = (q * NT + tid) * E;
+    if constexpr (ALN) V::store(yr, c, v[q]);
+    else store_any<T>(yr, c, cols, v[q]);
+  };
   // RMSNorm, GE: the weight g is loaded with the row, so its latency is not
   // exposed after the reduction.  8192^2 f32: 100.4 -> 91.6 us.  bf16 keeps
   // the load after the reduction: loaded early it costs VGPRs and waves per
   // SIMD (47.6 against 49.0 us packed, 52.9 us unpacked).
-  u32x4 graw[OP == ROW_RMSNORM ? VPT : 1];
-  if constexpr (OP == ROW_RMSNORM && GE) {
+  constexpr bool kEarly = OP == ROW_RMSNORM && GE && ALN;
+  u32x4 graw[kEarly ? VPT : 1];
+  if constexpr (kEarly) {
 #pragma unroll
     for (int q = 0; q < VPT; ++q)
-      if (ok[q])
-        graw[q] = *reinterpret_cast<const u32x4*>(static_cast<const T*>(a.g) + (int64_t)(q * kRowThreads + tid) * E);
+      if (ok[q]) graw[q] = *reinterpret_cast<const u32x4*>(static_cast<const T*>(a.g) + (q * NT + tid) * E);
   }
 
   if (OP == ROW_SOFTMAX) {
@@ -316,7 +396,7 @@ __global__ __launch_bounds__(kRowThreads) void row_cached_kernel(RowArgs a) {
       if (ok[q])
 #pragma unroll
         for (int e = 0; e < E; ++e) m = xmax(m, v[q][e]);
-    m = block_max(m, redf);
+    m = block_max<NW>(m, redf);
     float s = 0.f;
 #pragma unroll
     for (int q = 0; q < VPT; ++q)
@@ -330,7 +410,7 @@ __global__ __launch_bounds__(kRowThreads) void row_cached_kernel(RowArgs a) {
           v[q][e] = ex;
           s += ex;
         }
-    s = block_sum(s, redf);
+    s = block_sum<NW>(s, redf);
     if (V::bf16) s = bf16r(s);
     const float r = 1.0f / s;
     // bf16: y = r(e / s) with e / s the IEEE f32 quotient (XLA:CPU divides in
@@ -350,7 +430,7 @@ __global__ __launch_bounds__(kRowThreads) void row_cached_kernel(RowArgs a) {
             v[q][e] = v[q][e] * r;
           }
         }
-        V::store(a.y, base + (int64_t)(q * kRowThreads + tid) * E, v[q]);
+        store(q);
       }
   } else if (OP == ROW_RMSNORM) {
     float s = 0.f;
@@ -359,16 +439,24 @@ __global__ __launch_bounds__(kRowThreads) void row_cached_kernel(RowArgs a) {
       if (ok[q])
 #pragma unroll
         for (int e = 0; e < E; ++e) s += v[q][e] * v[q][e];
-    s = block_sum(s, redf);
+    s = block_sum<NW>(s, redf);
     const float r = rsqrtf(s / (float)a.cols + a.eps);
 #pragma unroll
     for (int q = 0; q < VPT; ++q)
       if (ok[q]) {
-        const int64_t c = (int64_t)(q * kRowThreads + tid) * E;
-        if constexpr (!GE) graw[q] = *reinterpret_cast<const u32x4*>(static_cast<const T*>(a.g) + c);
+        const int c = (q * NT + tid) * E;
+        if constexpr (ALN) {
+          const u32x4 w = kEarly ? graw[kEarly ? q : 0]
+                                 : *reinterpret_cast<const u32x4*>(static_cast<const T*>(a.g) + c);
 #pragma unroll
-        for (int e = 0; e < E; ++e) v[q][e] = v[q][e] * r * row_elem<T>(graw[q], e);
-        V::store(a.y, base + c, v[q]);
+          for (int e = 0; e < E; ++e) v[q][e] = v[q][e] * r * row_elem<T>(w, e);
+        } else {
+          float gv[E];
+          load_any<T>(static_cast<const T*>(a.g), c, cols, 0.f, gv);
+#pragma unroll
+          for (int e = 0; e < E; ++e) v[q][e] = v[q][e] * r * gv[e];
+        }
+        store(q);
       }
   } else if (OP == ROW_ARGMAX) {
     // Two passes over the cached row: the NaN-propagating row maximum m,
@@ -381,22 +469,22 @@ __global__ __launch_bounds__(kRowThreads) void row_cached_kernel(RowArgs a) {
       if (ok[q])
 #pragma unroll
         for (int e = 0; e < E; ++e) m = xmax(m, v[q][e]);
-    m = block_max(m, redf);
+    m = block_max<NW>(m, redf);
     int bi = 0x7FFFFFFF;
     if (m != m) {
 #pragma unroll
       for (int q = VPT - 1; q >= 0; --q)
         if (ok[q])
 #pragma unroll
-          for (int e = E - 1; e >= 0; --e) bi = v[q][e] != v[q][e] ? (q * kRowThreads + tid) * E + e : bi;
+          for (int e = E - 1; e >= 0; --e) bi = v[q][e] != v[q][e] ? (q * NT + tid) * E + e : bi;
     } else {
 #pragma unroll
       for (int q = VPT - 1; q >= 0; --q)
         if (ok[q])
 #pragma unroll
-          for (int e = E - 1; e >= 0; --e) bi = v[q][e] == m ? (q * kRowThreads + tid) * E + e : bi;
+          for (int e = E - 1; e >= 0; --e) bi = v[q][e] == m ? (q * NT + tid) * E + e : bi;
     }
-    bi = block_min_int(bi, redi);
+    bi = block_min_int<NW>(bi, redi);
     if (tid == 0) static_cast<int32_t*>(a.y)[row] = bi == 0x7FFFFFFF ? 0 : bi;
   } else if (OP == ROW_SUM) {
     float s = 0.f;
@@ -405,7 +493,7 @@ __global__ __launch_bounds__(kRowThreads) void row_cached_kernel(RowArgs a) {
       if (ok[q])
 #pragma unroll
         for (int e = 0; e < E; ++e) s += v[q][e];
-    s = block_sum(s, redf);
+    s = block_sum<NW>(s, redf);
     if (tid == 0) V::store1(a.y, row, s);
   } else {  // ROW_MAX, ROW_MIN
     const float sg = OP == ROW_MIN ? -1.f : 1.f;
@@ -415,38 +503,40 @@ __global__ __launch_bounds__(kRowThreads) void row_cached_kernel(RowArgs a) {
       if (ok[q])
 #pragma unroll
         for (int e = 0; e < E; ++e) m = xmax(m, sg * v[q][e]);
-    m = block_max(m, redf);
+    m = block_max<NW>(m, redf);
     if (tid == 0) V::store1(a.y, row, sg * m);
   }
   }
 }
 
-// Streaming row kernel for any cols: scalar strided passes over the row
-// (max / sums first, then the output pass re-reads the row).
+// Streaming row kernel for rows beyond the register cache (65536 f32 or
+// 131072 bf16 columns): strided passes over the row (max / sums first, then
+// the output pass re-reads the row).
 template <typename T, int OP>
-__global__ __launch_bounds__(kRowThreads) void row_stream_kernel(RowArgs a) {
+__global__ __launch_bounds__(kRowMaxThreads) void row_stream_kernel(RowArgs a) {
   using V = Vec<T>;
-  __shared__ float redf[4];
-  __shared__ int redi[4];
+  constexpr int NW = kRowMaxThreads / kWave;
+  __shared__ float redf[NW];
+  __shared__ int redi[NW];
   for (int64_t row = blockIdx.x; row < a.rows; row += gridDim.x) {
   const int64_t base = row * a.cols;
   const int tid = threadIdx.x;
   if (OP == ROW_SOFTMAX) {
     float m = -INFINITY;
-    for (int64_t c = tid; c < a.cols; c += kRowThreads) m = xmax(m, V::load1(a.x, base + c));
-    m = block_max(m, redf);
+    for (int64_t c = tid; c < a.cols; c += kRowMaxThreads) m = xmax(m, V::load1(a.x, base + c));
+    m = block_max<NW>(m, redf);
     float s = 0.f;
-    for (int64_t c = tid; c < a.cols; c += kRowThreads) {
+    for (int64_t c = tid; c < a.cols; c += kRowMaxThreads) {
       float d = V::load1(a.x, base + c) - m;
       if (V::bf16) d = bf16r(d);
       float ex = __expf(d);
       if (V::bf16) ex = bf16r(ex);
       s += ex;
     }
-    s = block_sum(s, redf);
+    s = block_sum<NW>(s, redf);
     if (V::bf16) s = bf16r(s);
     const float r = 1.0f / s;
-    for (int64_t c = tid; c < a.cols; c += kRowThreads) {
+    for (int64_t c = tid; c < a.cols; c += kRowMaxThreads) {
       float d = V::load1(a.x, base + c) - m;
       if (V::bf16) d = bf16r(d);
       float ex = __expf(d);
@@ -457,20 +547,20 @@ __global__ __launch_bounds__(kRowThreads) void row_stream_kernel(RowArgs a) {
     }
   } else if (OP == ROW_RMSNORM) {
     float s = 0.f;
-    for (int64_t c = tid; c < a.cols; c += kRowThreads) {
+    for (int64_t c = tid; c < a.cols; c += kRowMaxThreads) {
       const float x = V::load1(a.x, base + c);
       s += x * x;
     }
-    s = block_sum(s, redf);
+    s = block_sum<NW>(s, redf);
     const float r = rsqrtf(s / (float)a.cols + a.eps);
-    for (int64_t c = tid; c < a.cols; c += kRowThreads)
+    for (int64_t c = tid; c < a.cols; c += kRowMaxThreads)
       V::store1(a.y, base + c, V::load1(a.x, base + c) * r * V::load1(a.g, c));
   } else if (OP == ROW_ARGMAX) {
     float bv = -INFINITY;
     int bi = 0x7FFFFFFF;
     bool nan = false;
     int nan_i = 0x7FFFFFFF;
-    for (int64_t c = tid; c < a.cols; c += kRowThreads) {
+    for (int64_t c = tid; c < a.cols; c += kRowMaxThreads) {
       const float x = V::load1(a.x, base + c);
       if (x != x) {
         if (!nan) {
@@ -484,18 +574,18 @@ __global__ __launch_bounds__(kRowThreads) void row_stream_kernel(RowArgs a) {
     }
     float rv = nan ? NAN : bv;
     int ri = nan ? nan_i : bi;
-    block_argmax(rv, ri, redf, redi);
+    block_argmax<NW>(rv, ri, redf, redi);
     if (tid == 0) static_cast<int32_t*>(a.y)[row] = ri == 0x7FFFFFFF ? 0 : ri;
   } else if (OP == ROW_SUM) {
     float s = 0.f;
-    for (int64_t c = tid; c < a.cols; c += kRowThreads) s += V::load1(a.x, base + c);
-    s = block_sum(s, redf);
+    for (int64_t c = tid; c < a.cols; c += kRowMaxThreads) s += V::load1(a.x, base + c);
+    s = block_sum<NW>(s, redf);
     if (tid == 0) V::store1(a.y, row, s);
   } else {  // ROW_MAX, ROW_MIN
     const float sg = OP == ROW_MIN ? -1.f : 1.f;
     float m = -INFINITY;
-    for (int64_t c = tid; c < a.cols; c += kRowThreads) m = xmax(m, sg * V::load1(a.x, base + c));
-    m = block_max(m, redf);
+    for (int64_t c = tid; c < a.cols; c += kRowMaxThreads) m = xmax(m, sg * V::load1(a.x, base + c));
+    m = block_max<NW>(m, redf);
     if (tid == 0) V::store1(a.y, row, sg * m);
   }
   }
@@ -511,6 +601,7 @@ __global__ __launch_bounds__(kRowThreads) void row_stream_kernel(RowArgs a) {
 namespace {
 
 constexpr int64_t kMaxRowBlocks = 1 << 20;
+constexpr int64_t kManyRows = 512;
 
 // MK_ROW_WAVE=0 keeps argmax / max / min on the workgroup-per-row kernels
 // (same results).
@@ -548,15 +639,38 @@ hipError_t launch_row(const mk::RowArgs& a, hipStream_t st) {
       return hipGetLastError();
     }
   }
-  if (aligned && vpt <= 16) {
-    if (vpt <= 1) hipLaunchKernelGGL((mk::row_cached_kernel<T, OP, 1>), grid, block, 0, st, a);
-    else if (vpt <= 2) hipLaunchKernelGGL((mk::row_cached_kernel<T, OP, 2>), grid, block, 0, st, a);
-    else if (vpt <= 4) hipLaunchKernelGGL((mk::row_cached_kernel<T, OP, 4>), grid, block, 0, st, a);
-    else if (vpt <= 8) hipLaunchKernelGGL((mk::row_cached_kernel<T, OP, 8>), grid, block, 0, st, a);
-    else hipLaunchKernelGGL((mk::row_cached_kernel<T, OP, 16>), grid, block, 0, st, a);
-  } else {
-    hipLaunchKernelGGL((mk::row_stream_kernel<T, OP>), grid, block, 0, st, a);
+  // One wave a row for many short ones; 256 threads while the row fits
+  // their registers and is short or one of many; else 1024, while it fits
+  // (16 vectors of f32, 8 of bf16, whose 8 values each are unpacked).  Few rows:
+  // at 8 vectors of 256 threads 1024 gain nothing yet (16 x 8192 f32 softmax
+  // 3.4 / 3.5 us), at 16 they do (64 x 32000 bf16 8.8 / 6.9).
+  const int64_t vpt_max = (vecs + mk::kRowMaxThreads - 1) / mk::kRowMaxThreads;
+  const bool wave_rows = a.rows >= kManyRows && vecs <= 4 * mk::kWave;
+  const bool wide = vpt > 16 || (vpt > 8 && a.rows < kManyRows);
+  if (wide && vpt_max > (sizeof(T) == 4 ? 16 : 8)) {
+    hipLaunchKernelGGL((mk::row_stream_kernel<T, OP>), grid, dim3(mk::kRowMaxThreads), 0, st, a);
+    return hipGetLastError();
   }
+#define MK_ROW_LAUNCH(VPT, NT, THREADS, GRID)                                                                          \
+  if (aligned) hipLaunchKernelGGL((mk::row_cached_kernel<T, OP, VPT, NT, true>), GRID, dim3(THREADS), 0, st, a);       \
+  else hipLaunchKernelGGL((mk::row_cached_kernel<T, OP, VPT, NT, false>), GRID, dim3(THREADS), 0, st, a);
+  if (wave_rows) {
+    const dim3 wgrid((unsigned)std::min<int64_t>((a.rows + 3) / 4, kMaxRowBlocks));
+    if (vecs <= mk::kWave) { MK_ROW_LAUNCH(1, mk::kWave, mk::kRowThreads, wgrid) }
+    else if (vecs <= 2 * mk::kWave) { MK_ROW_LAUNCH(2, mk::kWave, mk::kRowThreads, wgrid) }
+    else { MK_ROW_LAUNCH(4, mk::kWave, mk::kRowThreads, wgrid) }
+  } else if (wide) {
+    if (vpt_max <= 4) { MK_ROW_LAUNCH(4, mk::kRowMaxThreads, mk::kRowMaxThreads, grid) }
+    else if (vpt_max <= 8) { MK_ROW_LAUNCH(8, mk::kRowMaxThreads, mk::kRowMaxThreads, grid) }
+    else if constexpr (sizeof(T) == 4) { MK_ROW_LAUNCH(16, mk::kRowMaxThreads, mk::kRowMaxThreads, grid) }
+  } else {
+    if (vpt <= 1) { MK_ROW_LAUNCH(1, mk::kRowThreads, mk::kRowThreads, grid) }
+    else if (vpt <= 2) { MK_ROW_LAUNCH(2, mk::kRowThreads, mk::kRowThreads, grid) }
+    else if (vpt <= 4) { MK_ROW_LAUNCH(4, mk::kRowThreads, mk::kRowThreads, grid) }
+    else if (vpt <= 8) { MK_ROW_LAUNCH(8, mk::kRowThreads, mk::kRowThreads, grid) }
+    else { MK_ROW_LAUNCH(16, mk::kRowThreads, mk::kRowThreads, grid) }
+  }
+#undef MK_ROW_LAUNCH
   return hipGetLastError();
 }
 
