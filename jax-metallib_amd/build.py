@@ -40,6 +40,7 @@ KERNEL_SOURCES = [
     "ew_jit.cpp",
     "kernels/qmatmul.hip",
     "kernels/qgemm.hip",
+    "kernels/qtile.hip",
     "kernels/decoder.hip",
     "kernels/gemm.hip",
     "kernels/gemm_tile.hip",

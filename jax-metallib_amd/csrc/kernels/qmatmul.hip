@@ -1527,6 +1527,8 @@ __global__ __launch_bounds__(256) void qmm_dequant_pair_kernel(QArgs g, QArgs u,
 // ---------------------------------------------------------------------------
 #include "../capi_internal.h"
 #include "qgemm.h"
+#include "gemm_tile.h"
+#include "qtile.h"
 
 namespace {
 
@@ -1543,6 +1545,8 @@ struct QPlan {
   int wide8_cs;      // its column split (1: every wave over all 256 columns; 2: halves)
   int deq;           // 1: dequantise W to bf16 in the workspace, then the bf16 GEMM
   int qg;            // 1: the many-row kernel of qgemm.hip (K split ks ways)
+  int qt;            // 1: the mid-row kernel of qtile.hip, as `tile` says
+  mkq::QTilePlan tile;
   size_t lds_bytes;
   int64_t part_bytes;
 };
@@ -1740,7 +1744,7 @@ constexpr int kDeqFallbackRows = 256;
 // qg_cap bounds the workspace the many-row kernel's K split may use (the
 // no-allocation entry point passes its array's size; the kernel then runs
 // unsplit rather than ask for more).
-bool plan_q(int fmt, int64_t M, int64_t K, int64_t N, QPlan* p, int64_t qg_cap = INT64_MAX) {
+bool plan_base(int fmt, int64_t M, int64_t K, int64_t N, QPlan* p, int64_t qg_cap = INT64_MAX) {
   *p = QPlan{};
   const int qg_m = env_int("MK_QMM_QG_M", kQgMinRows);
   const int deq_m = env_int("MK_QMM_DEQ_M", kDeqMinRows);
@@ -1794,6 +1798,57 @@ bool plan_q(int fmt, int64_t M, int64_t K, int64_t N, QPlan* p, int64_t qg_cap =
 done:
   p->part_bytes = p->ks > 1 ? (int64_t)mk::kWidePartOffset + (int64_t)p->rowblocks * p->ks * mk::kQRows * N * 4 : 0;
   return true;
+}
+
+// Estimated microseconds of a base plan, launch included, over the range in
+// which the mid-row kernel can stand in for it.  The rates are of the kernels
+// measured at K, N = 4096 x 14336, 4096 x 1792, 8192 x 8192, 1088 x 3008 and
+// 2048 x 5000, 17 to 1000 rows (within a fifth):
+//   * streaming kernels: 7.3e6 weights a us, counted once per 16 rows;
+//   * the 64-column kernel: 2.9e6, and 13.4 ns a k of a wave's serial share;
+//   * qgemm.hip: 0.95 us a 64-k step of a 256 x 128 tile, a round of 256 tiles;
+//   * dequantise, then GEMM: 2 bytes a weight at 4.3e6 a us, the GEMM as
+//     gemm_tile.hip estimates it.  A fifth off: that estimate is up to 8 %
+//     high and the mid-row kernel's, with several rounds of tiles, 15 % low.
+double base_estimate(const QPlan& p, int64_t M, int64_t K, int64_t N) {
+  if (p.qg) {
+    const double tiles = (double)((M + 255) / 256) * (N / 128) * p.ks, steps = (double)K / 64 / p.ks;
+    return 4.0 + std::ceil(tiles / 256) * steps * 0.95 + (p.ks > 1 ? 3.0 + p.part_bytes / 5.5e6 : 0.0);
+  }
+  if (p.deq) {
+    mkg::TileGemm g;
+    g.M = M;
+    g.N = N;
+    g.K = K;
+    g.lda = K;
+    g.ldb = N;
+    return 0.8 * (7.0 + 2.0 * K * N / 4.3e6 + mkg::tile_estimate(g, mkg::tile_pick(g)));
+  }
+  const double weights = (double)((M + mk::kQRows - 1) / mk::kQRows) * K * N;
+  if (p.wide_groups > 0 || p.wide8_steps > 0 || p.stream_steps > 0) return 3.5 + weights / 7.3e6;
+  return 3.5 + std::max(p.kwave * 0.0134, weights / 2.9e6);
+}
+
+// Takes the base plan *p to the mid-row kernel of qtile.hip where that is
+// estimated faster (M = 100, K = 4096, N = 14336: int8 66 -> 22 us, int4 57 ->
+// 28; M = 128, N = 1792: 37 -> 12 and 14; M = 700: int8 129 -> 91; M = 1, K =
+// 4032, N = 4096: int8 48 -> 11).  Not up to 16 rows where a streaming kernel
+// fits (int8 16 x 4096 x 14336: 15.4 us, this one 16.4); and not where the
+// dequantise-then-GEMM route has a paired SwiGLU form, so that two products
+// and the paired one keep the same bits.  MK_QMM_QT=0 turns it off, 2 takes
+// it wherever it can run (tests).
+void consider_qtile(int fmt, int64_t M, int64_t K, int64_t N, int64_t cap, QPlan* p) {
+  const bool streaming = p->wide_groups > 0 || p->wide8_steps > 0 || p->stream_steps > 0;
+  if (M <= mk::kQRows && streaming) return;
+  const int env = env_int("MK_QMM_QT", 1);
+  if (env == 0 || (env != 2 && p->deq && M % 256 == 0 && N % 128 == 0)) return;
+  mkq::QTilePlan t;
+  if (!mkq::qtile_plan(fmt == MK_QFMT_INT4_G64, M, K, N, cap, &t)) return;
+  if (env != 2 && t.us >= base_estimate(*p, M, K, N)) return;
+  *p = QPlan{};
+  p->qt = 1;
+  p->tile = t;
+  p->part_bytes = t.bytes;
 }
 
 // Kernels that need more than the default 64 KB of dynamic LDS must opt in.
@@ -1961,8 +2016,12 @@ int run_q(int fmt, const void* x, const void* w, const void* s, const void* z, v
   if (M > (1 << 20) || K > (1 << 24) || N > (1 << 26) || (M * K) > (int64_t)1 << 31)
     return mkc::fail(MK_EINVAL, "%s: shape too large", fn);
   QPlan p;
-  if (!plan_q(fmt, M, K, N, &p, qg_cap))
+  // The mid-row kernel's vector accesses want the tensors' own alignment; a
+  // pointer off it stays on the base plan.
+  const bool qt = epi != MK_EPI_SWIGLU_PAIRS && mkq::qtile_aligned(fmt == MK_QFMT_INT4_G64, x, w, s, z, y, aux, N);
+  if (!plan_base(fmt, M, K, N, &p, qg_cap))
     return mkc::fail(MK_EUNSUPPORTED, "%s: no launch configuration for K=%lld", fn, (long long)K);
+  if (qt) consider_qtile(fmt, M, K, N, qg_cap, &p);
   // The paired SwiGLU (interleaved gate / up columns, y [M, N/2]) is an
   // epilogue of the bf16 GEMM only: it needs the dequantise-then-GEMM route.
   if (epi == MK_EPI_SWIGLU_PAIRS && !p.deq)
@@ -1993,6 +2052,11 @@ int run_q(int fmt, const void* x, const void* w, const void* s, const void* z, v
   a.epi = epi;
   hipStream_t st = static_cast<hipStream_t>(stream);
   hipError_t e;
+  if (p.qt) {
+    e = mkq::qtile_launch(fmt == MK_QFMT_INT4_G64, x, w, s, z, y, M, K, N, aux, epi, p.tile, ws, st);
+    if (e != hipSuccess) return mkc::fail(MK_ELAUNCH, "%s: launch failed: %s", fn, hipGetErrorString(e));
+    return MK_OK;
+  }
   if (p.qg) {
     // The split-K exchange stays in one XCD's L2 when the placement probe
     // has seen round-robin dealing (as for the wide kernel below).
@@ -2081,9 +2145,12 @@ extern "C" int64_t mk_qmatmul_workspace_bytes(int fmt, int64_t M, int64_t K, int
   if ((fmt != MK_QFMT_INT4_G64 && fmt != MK_QFMT_INT8_PC) || M <= 0 || K <= 0 || N <= 0 ||
       K % 64 != 0)
     return -1;
+  // Enough for either plan: which one runs depends on the pointers as well.
   QPlan p;
-  if (!plan_q(fmt, M, K, N, &p)) return -1;
-  return p.part_bytes;
+  if (!plan_base(fmt, M, K, N, &p)) return -1;
+  const int64_t base = p.part_bytes;
+  consider_qtile(fmt, M, K, N, INT64_MAX, &p);
+  return std::max(p.part_bytes, base);
 }
 
 extern "C" int mk_qmatmul_epilogue_supported(int fmt, int64_t M, int64_t K, int64_t N, int epilogue) {
@@ -2091,7 +2158,7 @@ extern "C" int mk_qmatmul_epilogue_supported(int fmt, int64_t M, int64_t K, int6
   if (epilogue == MK_EPI_NONE || epilogue == MK_EPI_ADD || epilogue == MK_EPI_SWIGLU) return 1;
   if (epilogue != MK_EPI_SWIGLU_PAIRS) return 0;
   QPlan p;
-  return plan_q(fmt, M, K, N, &p) && p.deq && M % 256 == 0 && N % 256 == 0 ? 1 : 0;
+  return plan_base(fmt, M, K, N, &p) && p.deq && M % 256 == 0 && N % 256 == 0 ? 1 : 0;
 }
 
 extern "C" int mk_int4g64_matmul_bf16(const void* x, const void* w_packed, const void* scale,
@@ -2145,7 +2212,7 @@ int64_t pair_workspace(int fmt, int64_t M, int64_t K, int64_t N) {
       N % 128 != 0 || M % 256 != 0)
     return -1;
   QPlan p;
-  if (!plan_q(fmt, M, K, N, &p) || !p.deq) return -1;
+  if (!plan_base(fmt, M, K, N, &p) || !p.deq) return -1;
   return (int64_t)mk::kWidePartOffset + K * (2 * N) * 2;
 }
 
@@ -2268,11 +2335,11 @@ extern "C" int mk_int4g64_matmul_bf16_noalloc(const void* x, const void* w_packe
                                               const void* zero, void* y, int64_t M, int64_t K, int64_t N,
                                               void* stream) {
   mkc::clear_error();
-  // The plan this entry point runs: the many-row kernel's K split only when
-  // its partials fit the array.
+  // What the base plan needs decides what is refused (its K split only when
+  // the partials fit the array); run_q keeps any other plan within it too.
   QPlan cp;
   const int64_t need = (M > 0 && K > 0 && N > 0 && K % 64 == 0 &&
-                        plan_q(MK_QFMT_INT4_G64, M, K, N, &cp, kNoAllocScratchBytes))
+                        plan_base(MK_QFMT_INT4_G64, M, K, N, &cp, kNoAllocScratchBytes))
                            ? cp.part_bytes
                            : -1;
   if (need > kNoAllocScratchBytes)
