@@ -19,7 +19,11 @@
 //     registers, one barrier per step, (S - 1) steps in flight, which is
 //     what the small tiles live on (16 x 64: 60 KB in flight per workgroup).
 //     Pieces beyond K come from a zero page; rows and columns beyond M and N
-//     repeat valid ones, whose results are not stored.
+//     repeat valid ones, whose results are not stored.  The main loop has no
+//     branch per piece: with one, 256 rows of 4096 x 4096 on 64 x 64 tiles
+//     took 22.6 us, without it 16.8, 128 x 128 tiles 37.7 and 29.6.
+//   * 16-bit results go through LDS and leave in 16-byte pieces side by side
+//     (1000 x 14336 x 4096 on 256 x 256 tiles, with the loop: 115 -> 102 us).
 //   * Operands whose rows are not 16-byte aligned are fed through registers
 //     (unaligned 16-byte loads, double-buffered LDS, the next step's loads
 //     under this step's MFMAs).
@@ -83,40 +87,48 @@ __device__ __forceinline__ u32x4 keep8(const u32x4& v, int n) {
   return o;
 }
 
-// Four consecutive results of one row.
 template <bool F16>
-__device__ __forceinline__ void tile_store4(const TileArgs& p, int64_t zc, int m, int n, const f32x4& v) {
-  const int64_t off = zc + (int64_t)m * p.N + n;
-  const bool whole = n + 4 <= p.N;
-  if (p.out_f32) {
-    float* c = static_cast<float*>(p.c) + off;
-    if (whole) {
-      *reinterpret_cast<f32x4_u4*>(c) = v;
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (n + e < p.N) c[e] = v[e];
-    }
-    return;
-  }
-  uint16_t* c = static_cast<uint16_t*>(p.c) + off;
-  u32x2 o;
+__device__ __forceinline__ u32x2 tile_pack4(const f32x4& v) {
   if constexpr (F16) {
     auto h = [](float f) { return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)f); };
-    o = u32x2{h(v.x) | (h(v.y) << 16), h(v.z) | (h(v.w) << 16)};
+    return u32x2{h(v.x) | (h(v.y) << 16), h(v.z) | (h(v.w) << 16)};
   } else {
-    if (p.epi != MK_EPI_NONE) {  // N % 4 == 0
-      epi_store_bf16x4(static_cast<uint16_t*>(p.c), p.aux, p.epi, (size_t)off, v);
-      return;
-    }
-    o = u32x2{pack_bf16x2(v.x, v.y), pack_bf16x2(v.z, v.w)};
+    return u32x2{pack_bf16x2(v.x, v.y), pack_bf16x2(v.z, v.w)};
   }
-  if (whole) {
-    *reinterpret_cast<u32x2_u2*>(c) = o;
+}
+
+// Eight consecutive 16-bit results of one row; the epilogues start from the
+// rounded product, which is what v holds.
+template <bool F16>
+__device__ __forceinline__ void tile_store8(const TileArgs& p, int64_t zc, int m, int n, const u32x4& v) {
+  const int64_t off = zc + (int64_t)m * p.N + n;
+  uint16_t* c = static_cast<uint16_t*>(p.c) + off;
+  if (!F16 && p.epi != MK_EPI_NONE) {  // N % 4 == 0
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      if (n + 4 * h >= p.N) break;
+      const uint32_t a = v[2 * h], b = v[2 * h + 1];
+      epi_store_bf16x4(static_cast<uint16_t*>(p.c), p.aux, p.epi, (size_t)(off + 4 * h),
+                       f32x4{bf16_to_f32(a & 0xffffu), bf16_to_f32(a >> 16), bf16_to_f32(b & 0xffffu), bf16_to_f32(b >> 16)});
+    }
+  } else if (n + 8 <= p.N) {
+    *reinterpret_cast<u32x4_u2*>(c) = v;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      if (n + e < p.N) c[e] = (uint16_t)(v[e >> 1] >> (16 * (e & 1)));
+  }
+}
+
+// Four consecutive f32 results of one row.
+__device__ __forceinline__ void tile_store4(const TileArgs& p, int64_t zc, int m, int n, const f32x4& v) {
+  float* c = static_cast<float*>(p.c) + zc + (int64_t)m * p.N + n;
+  if (n + 4 <= p.N) {
+    *reinterpret_cast<f32x4_u4*>(c) = v;
   } else {
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-      if (n + e < p.N) c[e] = (uint16_t)(o[e >> 1] >> (16 * (e & 1)));
+      if (n + e < p.N) c[e] = v[e];
   }
 }
 
@@ -229,8 +241,12 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_tile_kernel(TileArgs p) 
 #pragma unroll
     for (int i = 0; i < TM; ++i) af[i] = read_a(smem, 0, i);
     int slot = 0;  // slot of step t
-    auto step = [&](auto parity, int t) {
+    // ALWAYS: step t + S exists, whole, and is issued during this one's last
+    // part (no branch per piece: the main loop).
+    auto step = [&](auto parity, auto always, int t) {
       constexpr int P = decltype(parity)::value;
+      constexpr bool ALWAYS = decltype(always)::value;
+      const bool more = ALWAYS || t + S < NS;
       const unsigned char* cur = smem + slot * STEP;
       const int slot_nx = slot + 1 == S ? 0 : slot + 1;
       const unsigned char* nxt = smem + slot_nx * STEP;
@@ -238,7 +254,6 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_tile_kernel(TileArgs p) 
 #pragma unroll
       for (int s = 0; s < KS; ++s) {
         const bool lastpart = s == KS - 1;
-        const bool more = t + S < NS;  // a step is issued during this one's last part
         if (lastpart) {
           __builtin_amdgcn_sched_barrier(0);
           // This wave's pieces of step t + 1 have landed and its fragments
@@ -246,13 +261,13 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_tile_kernel(TileArgs p) 
           // every wave: step t + 1 may be read, step t's slot refilled.
           // (After the last step the reads below take a stale slot; their
           // values are not used.)
-          if (t + S - 1 < NS) vm_wait(D * (S - 2));
+          if (ALWAYS || t + S - 1 < NS) vm_wait(D * (S - 2));
           else vm_wait(0);
           __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
           __builtin_amdgcn_s_barrier();
           asm volatile("" ::: "memory");
           __builtin_amdgcn_sched_barrier(0);
-          if (more) cut_k(t + S);
+          if (!ALWAYS && more) cut_k(t + S);
         }
         const unsigned char* from = lastpart ? nxt : cur;
         const int sn = lastpart ? 0 : s + 1;
@@ -273,16 +288,18 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_tile_kernel(TileArgs p) 
       }
       slot = slot_nx;
     };
-    if constexpr (KS % 2 == 0) {
-      for (int t = 0; t < NS; ++t) step(std::integral_constant<int, 0>{}, t);
-    } else {
-      int t = 0;
-      for (; t + 1 < NS; t += 2) {
-        step(std::integral_constant<int, 0>{}, t);
-        step(std::integral_constant<int, 1>{}, t + 1);
-      }
-      if (t < NS) step(std::integral_constant<int, 0>{}, t);
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, KS % 2>;  // B's register sets turn over KS times a step
+    int t = 0;
+    for (; t + 2 + S < NS; t += 2) {
+      step(I0{}, std::true_type{}, t);
+      step(I1{}, std::true_type{}, t + 1);
     }
+    for (; t + 1 < NS; t += 2) {
+      step(I0{}, std::false_type{}, t);
+      step(I1{}, std::false_type{}, t + 1);
+    }
+    if (t < NS) step(I0{}, std::false_type{}, t);
   } else {
     auto multiply = [&](const unsigned char* st) {
   #pragma unroll
@@ -359,6 +376,28 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_tile_kernel(TileArgs p) 
 
   // Epilogue (C^T fragments): this lane holds row m, columns n .. n + 3.
   const int64_t zc = (int64_t)blockIdx.z * p.sc;
+  if (!p.out_f32) {
+    // 16-bit results through LDS, so that a row leaves in 16-byte pieces side
+    // by side; the row padding spreads the writes over all banks.
+    constexpr int RS = BN + 16;
+    uint16_t* stage = reinterpret_cast<uint16_t*>(smem);
+    __syncthreads();  // every wave is done with the ring
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+        *reinterpret_cast<u32x2*>(stage + (wm * 16 * TM + 16 * i + (lane & 15)) * RS + wn * 16 * TN + 16 * j +
+                                  4 * (lane >> 4)) = tile_pack4<F16>(acc[i][j]);
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < (BM * BN / 8 + NW * 64 - 1) / (NW * 64); ++q) {
+      const int c = q * NW * 64 + tid, row = c / (BN / 8), col = 8 * (c % (BN / 8));
+      if (BM * BN / 8 < NW * 64 && row >= BM) break;  // the smallest tile has fewer pieces than threads
+      if (m0 + row < M && n0 + col < N)
+        tile_store8<F16>(p, zc, m0 + row, n0 + col, *reinterpret_cast<const u32x4*>(stage + row * RS + col));
+    }
+    return;
+  }
   const int mrow = m0 + wm * 16 * TM + (lane & 15), ncol = n0 + wn * 16 * TN + 4 * (lane >> 4);
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
@@ -367,7 +406,7 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_tile_kernel(TileArgs p) 
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
       const int n = ncol + 16 * j;
-      if (n < N) tile_store4<F16>(p, zc, m, n, acc[i][j]);
+      if (n < N) tile_store4(p, zc, m, n, acc[i][j]);
     }
   }
 }
@@ -383,7 +422,8 @@ constexpr int step_bytes(int bm, int bn, int ks) { return (bm + bn) * 64 * ks; }
 
 template <int BM, int BN, int WM, int WN, int KS, int S, bool AT, bool BT, bool F16, bool DMA>
 hipError_t launch(const mk::TileArgs& p, int64_t batch, hipStream_t st) {
-  constexpr size_t lds = (size_t)S * step_bytes(BM, BN, KS);
+  constexpr size_t ring = (size_t)S * step_bytes(BM, BN, KS), stage = (size_t)BM * (BN + 16) * 2;
+  constexpr size_t lds = ring > stage ? ring : stage;
   static_assert(lds <= 160 * 1024, "LDS");
   const void* fn = (const void*)mk::gemm_tile_kernel<BM, BN, WM, WN, KS, S, AT, BT, F16, DMA>;
   if (lds > 64 * 1024) {
@@ -432,22 +472,22 @@ constexpr int kBn[kTileShapes] = {64, 64, 64, 64, 128, 256};
 
 // us per 32 k of one tile: alone on the chip, with one on every CU, and per
 // tile and CU with several (two resident).  Measured at K = 4096, e.g. fed by
-// DMA, M x 4096: 16 rows 13.1 us (16 x 64; 64 x 64 18.5, 128 x 128 34.9),
-// 128 rows 14.2 (32 x 64; 16 x 64 22.1), 256 rows 20.6 (64 x 64; 32 x 64
-// 25.1, 128 x 64 26.0), 512 rows 28.5 (128 x 64; 64 x 64 32.1), 2000 rows
-// 65.0 (128 x 128; 128 x 64 78.7, 256 x 256 92.8), 4096 rows 113.4 (256 x
-// 256; 128 x 128 133.9).  Through registers (N = 4097): 16 rows 18.2 / 28.9 /
+// DMA, M x 4096: 16 rows 12.2 us (16 x 64; 64 x 64 13.9, 128 x 128 28.0),
+// 128 rows 13.8 (32 x 64; 16 x 64 21.4), 256 rows 16.8 (64 x 64; 32 x 64
+// 24.6, 128 x 64 21.5), 512 rows 25.1 (128 x 64; 64 x 64 32.2), 2000 rows
+// 59.9 (128 x 128; 128 x 64 77.1, 256 x 256 87.6), 4096 rows 105.2 (256 x
+// 256; 128 x 128 119.3).  Through registers (N = 4097): 16 rows 18.2 / 28.9 /
 // 50.0 (16 x 64 / 64 x 64 / 128 x 128), 512 rows 117 / 59.7 / 54.8.
 struct Rate {
   double alone, full, each;
 };
-constexpr Rate kDmaRate[kTileShapes] = {{0.095, 0.100, 0.062}, {0.103, 0.111, 0.086}, {0.142, 0.158, 0.125},
-                                        {0.185, 0.225, 0.170}, {0.270, 0.345, 0.262}, {0.670, 0.930, 0.930}};
+constexpr Rate kDmaRate[kTileShapes] = {{0.088, 0.095, 0.060}, {0.094, 0.100, 0.075}, {0.101, 0.123, 0.112},
+                                        {0.142, 0.188, 0.165}, {0.210, 0.280, 0.235}, {0.590, 0.790, 0.790}};
 constexpr Rate kRegRate[kTileShapes] = {{0.148, 0.155, 0.109}, {1e9, 1e9, 1e9}, {0.225, 0.240, 0.175},
                                         {1e9, 1e9, 1e9}, {0.400, 0.490, 0.370}, {1e9, 1e9, 1e9}};
 // us a CU spends on a tile besides: the first step's latency and the stores,
 // half hidden where two workgroups share the CU.
-constexpr double kTileOver[kTileShapes] = {0.1, 0.2, 0.3, 0.6, 1.2, 8.0};
+constexpr double kTileOver[kTileShapes] = {0.1, 0.2, 0.3, 0.6, 1.2, 5.5};
 
 }  // namespace
 

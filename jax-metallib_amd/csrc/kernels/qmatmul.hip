@@ -1808,8 +1808,8 @@ done:
 //   * the 64-column kernel: 2.9e6, and 13.4 ns a k of a wave's serial share;
 //   * qgemm.hip: 0.95 us a 64-k step of a 256 x 128 tile, a round of 256 tiles;
 //   * dequantise, then GEMM: 2 bytes a weight at 4.3e6 a us, the GEMM as
-//     gemm_tile.hip estimates it.  A fifth off: that estimate is up to 8 %
-//     high and the mid-row kernel's, with several rounds of tiles, 15 % low.
+//     gemm_tile.hip estimates it.  A fifth off: the mid-row kernel's own
+//     estimate is up to that low with several rounds of tiles.
 double base_estimate(const QPlan& p, int64_t M, int64_t K, int64_t N) {
   if (p.qg) {
     const double tiles = (double)((M + 255) / 256) * (N / 128) * p.ks, steps = (double)K / 64 / p.ks;
@@ -1822,7 +1822,7 @@ double base_estimate(const QPlan& p, int64_t M, int64_t K, int64_t N) {
     g.K = K;
     g.lda = K;
     g.ldb = N;
-    return 0.8 * (7.0 + 2.0 * K * N / 4.3e6 + mkg::tile_estimate(g, mkg::tile_pick(g)));
+    return 0.78 * (7.0 + 2.0 * K * N / 4.3e6 + mkg::tile_estimate(g, mkg::tile_pick(g)));
   }
   const double weights = (double)((M + mk::kQRows - 1) / mk::kQRows) * K * N;
   if (p.wide_groups > 0 || p.wide8_steps > 0 || p.stream_steps > 0) return 3.5 + weights / 7.3e6;
