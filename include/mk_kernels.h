@@ -60,7 +60,8 @@ const char* mk_version(void);
  * partial sums when a call splits K across workgroups, and for many rows
  * (M >= 768, or M >= 256 when N % 64 != 0) the bf16-dequantised W [K, N]
  * that the bf16 GEMM then multiplies; mk_qmatmul_workspace_bytes gives the
- * size, 0 when none is needed (then workspace may be NULL).  Its first 64 KB hold per-tile arrival counters:
+ * size that is enough for every route of the shape, 0 when none is needed
+ * (then workspace may be NULL).  Its first 64 KB hold per-tile arrival counters:
  * zero-fill a workspace once before its first use; every completed call
  * leaves the counters at zero again.  Calls that share a workspace must be
  * ordered (same stream).
@@ -124,9 +125,9 @@ int mk_int8pc_matmul_swiglu_pair_bf16(const void* x, const void* wg, const void*
  * cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc).  No counterpart in the reference.
  * The workspace is a file-scope device array of 8 MiB per GPU, held until the
- * process ends.  The many-row kernel (128 <= M < 768) runs here without its
- * K split when the split's partials would not fit (at K = 4096, N = 14336:
- * same results to the bf16 tolerance, not bit for bit); shapes whose plan
+ * process ends.  The mid- and many-row kernels (M > 16) run here with the
+ * K split whose partials fit, or none (M = 256, K = 4096, N = 14336: same
+ * results to the bf16 tolerance, not bit for bit); shapes whose plan
  * still needs more than 8 MiB (the dequantise-then-GEMM route, for example
  * M >= 768 at K = 4096, N = 14336) return MK_EWORKSPACE before any launch.
  * The first call on a device sets the array up (its address, and its

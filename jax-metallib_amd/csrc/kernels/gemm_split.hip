@@ -27,9 +27,10 @@
 //     with none, the smallest kept product is at least 2^-114 and nothing was
 //     lost; with one, the tile is recomputed.
 //
-// Layout: operands go through registers (f32 loads of 4-byte alignment, two
-// steps ahead of the MFMAs), are split there and staged as three bf16 planes
-// in the order and swizzle of the 16-bit tile family, double buffered.  8
+// Layout: operands go through registers (f32 loads of 4-byte alignment, one
+// step ahead of the MFMAs, two for 16-row tiles), are split there and staged
+// as three bf16 planes in the order and swizzle of the 16-bit tile family,
+// double buffered.  8
 // waves (128 x 128), two to a SIMD, so that one's splitting runs under the
 // other's MFMAs.
 #include "common.h"
