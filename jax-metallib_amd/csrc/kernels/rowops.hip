@@ -129,8 +129,8 @@ struct Vec<uint16_t> {
 // one wave).  With 16 waves each combines the partials by another shuffle.
 template <int NW>
 __device__ __forceinline__ float block_sum(float v, float* red) {
+  static_assert(NW > 1, "one wave: wave_row_sum");
   v = wave_sum(v);
-  if constexpr (NW == 1) return v;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   __syncthreads();
   if (lane == 0) red[wv] = v;
@@ -140,6 +140,45 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
 #pragma unroll
   for (int o = NW / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   return v;
+}
+
+// The sum of a row held by one wave, vector 64 q + lane's own sum in v[q]: the
+// order of a workgroup's four waves of one vector a thread (a wave of zeros
+// where the row has fewer), so that a row's bits do not depend on which of the
+// two kernels has it.
+//
+// The VPT butterflies share their shuffles: at the first steps a lane hands
+// over the values that the other half goes on with (4 vectors: 7 shuffles
+// instead of 24; 8192 x 2048 bf16 sum 9.0 -> 8.1 us).
+template <int VPT>
+__device__ __forceinline__ float wave_row_sum(const float (&v)[VPT]) {
+  static_assert(VPT == 1 || VPT == 2 || VPT == 4, "the waves of a workgroup");
+  if constexpr (VPT == 1) return wave_sum(v[0]);
+  const int lane = threadIdx.x & 63;
+  const bool hi = lane & 32;
+  float s;
+  if constexpr (VPT == 2) {
+    s = (hi ? v[1] : v[0]) + __shfl_xor(hi ? v[0] : v[1], 32, 64);
+    s += __shfl_xor(s, 16, 64);
+  } else {
+    const float a = (hi ? v[2] : v[0]) + __shfl_xor(hi ? v[0] : v[2], 32, 64);
+    const float b = (hi ? v[3] : v[1]) + __shfl_xor(hi ? v[1] : v[3], 32, 64);
+    const bool odd = lane & 16;
+    s = (odd ? b : a) + __shfl_xor(odd ? a : b, 16, 64);
+  }
+#pragma unroll
+  for (int o = 8; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+  float sum = __shfl(s, 0, 64);
+#pragma unroll
+  for (int q = 1; q < VPT; ++q) sum += __shfl(s, q * (kWave / VPT), 64);
+  return sum;
+}
+
+// A row's sum from each thread's own: one value, or one per vector (NW 1).
+template <int NW, int NP>
+__device__ __forceinline__ float row_sum(const float (&v)[NP], float* red) {
+  if constexpr (NW == 1) return wave_row_sum(v);
+  else return block_sum<NW>(v[0], red);
 }
 
 template <int NW>
@@ -349,6 +388,7 @@ template <typename T, int OP, int VPT, int NT, bool ALN, bool GE = sizeof(T) == 
 __global__ __launch_bounds__(NT < kRowThreads ? kRowThreads : NT) void row_cached_kernel(RowArgs a) {
   using V = Vec<T>;
   constexpr int E = V::N, NW = NT / kWave, RPB = NT < kRowThreads ? kRowThreads / NT : 1;
+  constexpr int NP = NW == 1 ? VPT : 1;  // partial sums a thread keeps (wave_row_sum)
   constexpr float kFill = OP == ROW_RMSNORM || OP == ROW_SUM ? 0.f : OP == ROW_MIN ? INFINITY : -INFINITY;
   __shared__ float redf[NW];
   __shared__ int redi[NW];
@@ -397,7 +437,7 @@ __global__ __launch_bounds__(NT < kRowThreads ? kRowThreads : NT) void row_cache
 #pragma unroll
         for (int e = 0; e < E; ++e) m = xmax(m, v[q][e]);
     m = block_max<NW>(m, redf);
-    float s = 0.f;
+    float part[NP] = {};
 #pragma unroll
     for (int q = 0; q < VPT; ++q)
       if (ok[q])
@@ -408,9 +448,9 @@ __global__ __launch_bounds__(NT < kRowThreads ? kRowThreads : NT) void row_cache
           float ex = __expf(d);
           if (V::bf16) ex = bf16r(ex);
           v[q][e] = ex;
-          s += ex;
+          part[NP > 1 ? q : 0] += ex;
         }
-    s = block_sum<NW>(s, redf);
+    float s = row_sum<NW>(part, redf);
     if (V::bf16) s = bf16r(s);
     const float r = 1.0f / s;
     // bf16: y = r(e / s) with e / s the IEEE f32 quotient (XLA:CPU divides in
@@ -433,13 +473,18 @@ __global__ __launch_bounds__(NT < kRowThreads ? kRowThreads : NT) void row_cache
         store(q);
       }
   } else if (OP == ROW_RMSNORM) {
-    float s = 0.f;
+    float part[NP] = {};
 #pragma unroll
     for (int q = 0; q < VPT; ++q)
       if (ok[q])
 #pragma unroll
-        for (int e = 0; e < E; ++e) s += v[q][e] * v[q][e];
-    s = block_sum<NW>(s, redf);
+        for (int e = 0; e < E; ++e) {
+          float& p = part[NP > 1 ? q : 0];
+          // (Spelled out, or each instance contracts the first in its own way.)
+          if (e > 1 || (NP == 1 && q > 0)) p = __builtin_fmaf(v[q][e], v[q][e], p);
+          else if (e == 1) p = __builtin_fmaf(v[q][0], v[q][0], v[q][1] * v[q][1]);
+        }
+    const float s = row_sum<NW>(part, redf);
     const float r = rsqrtf(s / (float)a.cols + a.eps);
 #pragma unroll
     for (int q = 0; q < VPT; ++q)
@@ -487,13 +532,13 @@ __global__ __launch_bounds__(NT < kRowThreads ? kRowThreads : NT) void row_cache
     bi = block_min_int<NW>(bi, redi);
     if (tid == 0) static_cast<int32_t*>(a.y)[row] = bi == 0x7FFFFFFF ? 0 : bi;
   } else if (OP == ROW_SUM) {
-    float s = 0.f;
+    float part[NP] = {};
 #pragma unroll
     for (int q = 0; q < VPT; ++q)
       if (ok[q])
 #pragma unroll
-        for (int e = 0; e < E; ++e) s += v[q][e];
-    s = block_sum<NW>(s, redf);
+        for (int e = 0; e < E; ++e) part[NP > 1 ? q : 0] += v[q][e];
+    const float s = row_sum<NW>(part, redf);
     if (tid == 0) V::store1(a.y, row, s);
   } else {  // ROW_MAX, ROW_MIN
     const float sg = OP == ROW_MIN ? -1.f : 1.f;
@@ -509,8 +554,8 @@ __global__ __launch_bounds__(NT < kRowThreads ? kRowThreads : NT) void row_cache
   }
 }
 
-// Streaming row kernel for rows beyond the register cache (65536 f32 or
-// 131072 bf16 columns): strided passes over the row (max / sums first, then
+// Streaming row kernel for rows beyond the register cache (65536
+// columns): strided passes over the row (max / sums first, then
 // the output pass re-reads the row).
 template <typename T, int OP>
 __global__ __launch_bounds__(kRowMaxThreads) void row_stream_kernel(RowArgs a) {
@@ -613,6 +658,10 @@ bool row_wave_enabled() {
 template <typename T, int OP>
 hipError_t launch_row(const mk::RowArgs& a, hipStream_t st) {
   constexpr int E = mk::Vec<T>::N;
+  // bf16 with an output: a lane of a 2048-column row unpacks and writes 32
+  // values, which 256 threads do faster (aligned softmax 32768 x 2048, wave /
+  // 256: 55.0 / 46.0 us, 1024 x 2048 4.8 / 4.1; RMSNorm 48.0 / 45.5, 4.7 / 3.9).
+  constexpr bool kTwoPass = sizeof(T) == 2 && (OP == mk::ROW_SOFTMAX || OP == mk::ROW_RMSNORM);
   const bool aligned = a.cols % E == 0 && ((uintptr_t)a.x % 16 == 0) && ((uintptr_t)a.y % 16 == 0 || OP >= mk::ROW_ARGMAX) &&
                        (OP != mk::ROW_RMSNORM || (uintptr_t)a.g % 16 == 0);
   const int64_t vecs = (a.cols + E - 1) / E;
@@ -639,14 +688,23 @@ hipError_t launch_row(const mk::RowArgs& a, hipStream_t st) {
       return hipGetLastError();
     }
   }
-  // One wave a row for many short ones; 256 threads while the row fits
-  // their registers and is short or one of many; else 1024, while it fits
-  // (16 vectors of f32, 8 of bf16, whose 8 values each are unpacked).  Few rows:
-  // at 8 vectors of 256 threads 1024 gain nothing yet (16 x 8192 f32 softmax
-  // 3.4 / 3.5 us), at 16 they do (64 x 32000 bf16 8.8 / 6.9).
+  // One wave a row for many short ones; 256 threads while the row fits their
+  // registers (16 vectors of f32, 8 of bf16, whose 8 values each are
+  // unpacked); else 1024, while it fits theirs.
+  //
+  // A sum's order, and with it a row's last bit, depends on the row's length
+  // alone: the number of rows decides only between a wave and 256 threads,
+  // which add in the same order, and for argmax, max and min, which have no
+  // order.  Rows of 9 to 16 vectors a thread, 256 / 1024 threads (us): f32
+  // 4096 x 10000 sum 27.1 / 29.7, softmax 59.2 / 57.1, 64 x 16384 4.9 / 5.0;
+  // unaligned softmax 64 x 12001 5.4 / 4.7, 600 x 12001 12.2 / 14.4, RMSNorm
+  // 6.6 / 4.5 and 17.6 / 13.4, sum 4096 x 12001 33.7 / 37.9; bf16 64 x 32000
+  // RMSNorm 10.9 / 5.4, 4096 x 32768 softmax 117.6 / 101.5, argmax 165 / 78.
   const int64_t vpt_max = (vecs + mk::kRowMaxThreads - 1) / mk::kRowMaxThreads;
-  const bool wave_rows = a.rows >= kManyRows && vecs <= 4 * mk::kWave;
-  const bool wide = vpt > 16 || (vpt > 8 && a.rows < kManyRows);
+  const bool wave_rows = a.rows >= kManyRows && vecs <= (kTwoPass && aligned ? 2 : 4) * mk::kWave;
+  constexpr bool kNoSum = OP == mk::ROW_ARGMAX || OP == mk::ROW_MAX || OP == mk::ROW_MIN;
+  const bool wide = vpt > 16 || (vpt > 8 && (sizeof(T) == 2 || (kNoSum ? a.rows < kManyRows
+                                                                       : OP != mk::ROW_SUM && a.cols % E != 0)));
   if (wide && vpt_max > (sizeof(T) == 4 ? 16 : 8)) {
     hipLaunchKernelGGL((mk::row_stream_kernel<T, OP>), grid, dim3(mk::kRowMaxThreads), 0, st, a);
     return hipGetLastError();
@@ -668,7 +726,7 @@ hipError_t launch_row(const mk::RowArgs& a, hipStream_t st) {
     else if (vpt <= 2) { MK_ROW_LAUNCH(2, mk::kRowThreads, mk::kRowThreads, grid) }
     else if (vpt <= 4) { MK_ROW_LAUNCH(4, mk::kRowThreads, mk::kRowThreads, grid) }
     else if (vpt <= 8) { MK_ROW_LAUNCH(8, mk::kRowThreads, mk::kRowThreads, grid) }
-    else { MK_ROW_LAUNCH(16, mk::kRowThreads, mk::kRowThreads, grid) }
+    else if constexpr (sizeof(T) == 4) { MK_ROW_LAUNCH(16, mk::kRowThreads, mk::kRowThreads, grid) }
   }
 #undef MK_ROW_LAUNCH
   return hipGetLastError();

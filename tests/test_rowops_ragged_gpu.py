@@ -66,3 +66,23 @@ def test_ragged_rows_special_values(shape):
         y = ops.softmax(d).float().cpu().numpy()
         m = h.max(-1)
         np.testing.assert_array_equal(np.isnan(y).all(-1), ~np.isfinite(m), err_msg=dt)
+
+
+# Row lengths of each kernel that the number of rows chooses between: a wave or
+# 256 threads (up to 256 vectors), 256 or 1024 threads (above 8 vectors each).
+@pytest.mark.parametrize("dt,cols", [(dt, c) for dt in ("f32", "bf16") for c in (
+    100, 250, 256, 500, 512, 1000, 1024, 1025, 2048, 8200, 9001, 12000, 16384, 16400, 20001, 32000, 32768)])
+def test_a_rows_bits_do_not_depend_on_the_number_of_rows(dt, cols):
+    """Sums of a row are added in an order that its length alone decides."""
+    ops = _ops()
+    x, g = _x((600, cols), cols), _x((cols,), 1)
+    if dt == "bf16":
+        x, g = dev_bf16(obf.f32_to_bf16_bits(x)), dev_bf16(obf.f32_to_bf16_bits(g))
+    else:
+        x, g = dev(x), dev(g)
+    print(f"[rows bits] {dt} {cols}", flush=True)
+    for name, f in (("softmax", ops.softmax), ("rmsnorm", lambda v: ops.rmsnorm(v, g)),
+                    ("sum", lambda v: ops.reduce_lastdim(v, "sum"))):
+        many = f(x)
+        for n in (1, 7, 511):
+            assert torch.equal(f(x[:n].contiguous()), many[:n]), (name, n)
