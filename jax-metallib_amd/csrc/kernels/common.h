@@ -93,10 +93,12 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p) {
 // 16-byte LDS DMA of every lane (source per lane) to LDS byte address
 // lds_base + 16 * lane (lds_base wave-uniform), from inline asm: the
 // compiler does not see it, so it adds no vmcnt(0) before LDS accesses; the
-// caller waits with vm_wait (below) and a barrier.
+// caller waits with vm_wait (below) and a barrier.  Nor does it see that an
+// LDS DMA needs one wait state after a scalar write of M0, hence the s_nop.
 __device__ __forceinline__ void dma16_asm(const void* src, uint32_t lds_base) {
   const uint32_t base = __builtin_amdgcn_readfirstlane(lds_base);
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(base) : "memory");
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(base)
+               : "m0", "memory");
 }
 
 // s_waitcnt vmcnt(n) for a value the unrolled loops fold to a constant.

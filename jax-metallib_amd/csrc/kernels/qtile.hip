@@ -67,19 +67,23 @@ __device__ __forceinline__ u32x2 read_tr8(const unsigned char* p) {
   return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_qt_ptr)(p)));
 }
 
-// LDS DMA of 16 (4) bytes a lane from base + off to lds_base + 16 (4) * lane.
+// LDS DMA of 16 (4) bytes a lane from base + off to lds_base + 16 (4) * lane
+// (the s_nop: see dma16_asm).
 __device__ __forceinline__ void dma16_sbase(const void* base, uint32_t off, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds_base) : "memory");
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds_base)
+               : "m0", "memory");
 }
 
 __device__ __forceinline__ void dma4_sbase(const void* base, uint32_t off, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "s"(lds_base) : "memory");
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "s"(lds_base)
+               : "m0", "memory");
 }
 
 // 4-byte LDS DMA of every lane to lds_base + 4 * lane (see dma16_asm).
 __device__ __forceinline__ void dma4_asm(const void* src, uint32_t lds_base) {
   const uint32_t base = __builtin_amdgcn_readfirstlane(lds_base);
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dword %0, off" ::"v"(src), "s"(base) : "memory");
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(src), "s"(base)
+               : "m0", "memory");
 }
 
 // Signed bytes 2d and 2d + 1 of w -> a pair of bf16, exactly.
