@@ -20,6 +20,7 @@
 // The rest -- integers, short sums, strides that leave no contiguous
 // dimension -- has one thread per output element, grid-stride.
 #include "common.h"
+#include "dot_general.h"
 #include "gemm_split.h"
 #include "gemm_tile.h"
 
@@ -119,32 +120,21 @@ bool operand_order(int64_t sx, int64_t sk, int64_t X, int64_t K, bool* x_contigu
   return false;
 }
 
-// How the tiled kernels read the product's operands, if they do.  Short sums
-// stay on the thread-per-output kernel: below 16 most of a 32-k step is
-// padding.
-bool tile_form(const mk::DotArgs& p, mkg::TileGemm* g) {
-  if (p.K < 16) return false;
-  const int64_t top = (int64_t)1 << 30;
-  if (p.M > top || p.N > top || p.K > top || p.batch > 65535 || ((p.M + 15) / 16) * ((p.N + 63) / 64) > INT32_MAX)
-    return false;
-  bool n_contiguous = false;
-  if (!operand_order(p.sa[1], p.sa[2], p.M, p.K, &g->a_t, &g->lda) ||
-      !operand_order(p.sb[2], p.sb[1], p.N, p.K, &n_contiguous, &g->ldb))
-    return false;
-  g->b_t = !n_contiguous;
-  g->a = p.a;
-  g->b = p.b;
-  g->c = p.c;
-  g->batch = p.batch;
-  g->M = p.M;
-  g->N = p.N;
-  g->K = p.K;
-  g->sa = p.sa[0];
-  g->sb = p.sb[0];
-  return true;
-}
-
-hipError_t launch_tiled(mkg::TileGemm g, int type, int out_type, hipStream_t st) {
+hipError_t launch_tiled(const mk::DotArgs& p, const mkg::DotOrder& o, int type, int out_type, hipStream_t st) {
+  mkg::TileGemm g;
+  g.a = p.a;
+  g.b = p.b;
+  g.c = p.c;
+  g.batch = p.batch;
+  g.M = p.M;
+  g.N = p.N;
+  g.K = p.K;
+  g.lda = o.lda;
+  g.ldb = o.ldb;
+  g.sa = p.sa[0];
+  g.sb = p.sb[0];
+  g.a_t = o.a_t;
+  g.b_t = o.b_t;
   if (type == mk::kF32) {
     mkg::SplitGemm s;
     s.a = static_cast<const float*>(g.a);
@@ -169,6 +159,24 @@ hipError_t launch_tiled(mkg::TileGemm g, int type, int out_type, hipStream_t st)
 
 }  // namespace
 
+namespace mkg {
+
+// Short sums stay on the thread-per-output kernel: below 16 most of a 32-k
+// step is padding.
+bool dot_tiled(int64_t batch, int64_t M, int64_t N, int64_t K, const int64_t* sa, const int64_t* sb, DotOrder* o) {
+  if (K < 16) return false;
+  const int64_t top = (int64_t)1 << 30;
+  if (M > top || N > top || K > top || batch > 65535 || ((M + 15) / 16) * ((N + 63) / 64) > INT32_MAX) return false;
+  bool n_contiguous = false;
+  if (!operand_order(sa[1], sa[2], M, K, &o->a_t, &o->lda) ||
+      !operand_order(sb[2], sb[1], N, K, &n_contiguous, &o->ldb))
+    return false;
+  o->b_t = !n_contiguous;
+  return true;
+}
+
+}  // namespace mkg
+
 extern "C" int mk_dot_general(int type_a, int type_b, int type_out, const void* a, const void* b, void* c,
                               int64_t batch, int64_t M, int64_t N, int64_t K, const int64_t* a_strides,
                               const int64_t* b_strides, void* stream) {
@@ -192,9 +200,9 @@ extern "C" int mk_dot_general(int type_a, int type_b, int type_out, const void* 
   p.batch = batch; p.M = M; p.N = N; p.K = K;
   for (int i = 0; i < 3; ++i) { p.sa[i] = a_strides[i]; p.sb[i] = b_strides[i]; }
   p.out_type = type_out;
-  mkg::TileGemm g;
-  if (floats && tile_form(p, &g)) {
-    const hipError_t te = launch_tiled(g, type_a, type_out, static_cast<hipStream_t>(stream));
+  mkg::DotOrder order;
+  if (floats && mkg::dot_tiled(batch, M, N, K, p.sa, p.sb, &order)) {
+    const hipError_t te = launch_tiled(p, order, type_a, type_out, static_cast<hipStream_t>(stream));
     if (te != hipSuccess) return mkc::fail(MK_ELAUNCH, "%s: launch failed: %s", fn, hipGetErrorString(te));
     return MK_OK;
   }

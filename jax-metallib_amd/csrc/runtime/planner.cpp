@@ -32,6 +32,7 @@
 #include <stdexcept>
 #include <tuple>
 
+#include "../kernels/dot_general.h"
 #include "mk_runtime.h"
 
 namespace mkrt {
@@ -1094,11 +1095,12 @@ class Planner {
     const bool fast = !(general && gd.transposed) && dot_shape(op, &d) && fast_types && d.K > 0 &&
                       d.K % 8 == 0 && d.N % 8 == 0 && numel(v) == d.batch * d.M * d.N;
     // An lhs stored [K, M] (a weight gradient x^T dy) is read in place by the
-    // tiled kernels behind mk_dot_general; so is an rhs stored [N, K] from
-    // 2^27 multiply-adds where the GEMM below would copy it (smaller products
-    // keep the copy).
+    // tiled kernels behind mk_dot_general, if they take the other operand too;
+    // so is an rhs stored [N, K] from 2^27 multiply-adds where the GEMM below
+    // would copy it (smaller products keep the copy).
+    mkg::DotOrder order;
     const bool in_place =
-        general && !gd.copy_a && !gd.copy_b && gd.K >= 16 && gd.batch <= 65535 &&
+        general && !gd.copy_a && !gd.copy_b && mkg::dot_tiled(gd.batch, gd.M, gd.N, gd.K, gd.sa, gd.sb, &order) &&
         ((gd.sa[1] == 1 && gd.sa[2] >= gd.M && gd.M > 1) ||
          (gd.sb[1] == 1 && gd.sb[2] >= gd.K &&
           (ta == DT_F32 || gd.M % 256 != 0 || gd.N % 256 != 0 || gd.K % 32 != 0) &&
