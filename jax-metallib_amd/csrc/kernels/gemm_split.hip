@@ -1,9 +1,11 @@
 // f32 GEMM for gfx950 on the bf16 matrix cores.
 //
-// The f32 MFMA (16x16x4) has 1/16 of the bf16 MFMA's rate.  Every f32 value
-// is the sum of three bf16 values, x = x1 + x2 + x3 (8 significant bits
-// each, by rounding to nearest and taking the rest), exactly, as long as x3
-// does not underflow.  So a product is nine bf16 products, of which the three
+// The f32 MFMA (16x16x4) has 1/16 of the bf16 MFMA's rate.  The split into
+// bf16 parts is that of Henry, Tang and Heinecke ("Leveraging the bfloat16
+// Artificial Intelligence Datatype For Higher-Precision Computations", 2019):
+// every f32 value is the sum of three bf16 values, x = x1 + x2 + x3 (8
+// significant bits each, by rounding to nearest and taking the rest), exactly,
+// as long as x3 does not underflow.  So a product is nine bf16 products, of which the three
 // smallest (x2 y3, x3 y2, x3 y3: at most 2^-24 of it) are below half an ulp of
 // f32; the other six, each exact, are summed in f32 by six bf16 MFMAs of 32 k
 // where the f32 MFMA needs eight of 4 k, at 3/8 of their time.  The five
@@ -16,23 +18,33 @@
 // the MFMAs each changed nothing), 4096^3 1183 -> 751, 1024^3 33 -> 27,
 // 1000 x 3000 x 1000 86 -> 50.
 //
-// What the split cannot represent is recomputed by the f32 MFMA, tile by
-// tile, in the same launch (native()):
-//   * an infinity, a NaN or a value that rounds to a bf16 infinity: every
-//     such operand leaves a non-finite result, which is looked for at the end;
-//   * underflow of the small parts.  Parts lost at 2^-126 are beneath the
-//     rounding of a result of at least 2^-60 if no operand exceeds 2^18 (2^24
-//     terms).  A tile with a smaller result (zeros among them) or a larger
-//     operand has its operands read once more for a nonzero one below 2^-45;
-//     with none, the smallest kept product is at least 2^-114 and nothing was
-//     lost; with one, the tile is recomputed.
+// What the split cannot represent is recomputed by the f32 MFMA in the same
+// launch.  Each result decides for itself, from the largest and the smallest
+// nonzero magnitude of its row of A and of its column of B, so its bits are
+// those of any tile and whatever else the tile holds:
+//   * an infinity, a NaN or a value that rounds to a bf16 infinity leaves a
+//     non-finite result: recomputed;
+//   * what is below 2^-126 may be lost: parts (2^-125 of an operand) and
+//     products and sums of parts (2^-123 a term).  Nothing that counts is if
+//     the result is at least K 2^-96 times the larger of 1 and the largest
+//     magnitudes (all K losses together are below 2^-26 of it), if the row or
+//     the column is all zeros, or if their smallest magnitudes are at least
+//     2^-100 (all parts are kept) and have a product of at least 2^-96 (a loss
+//     is below 2^-27 of its own term).  Else: recomputed.
+// The largest magnitudes are kept while the operands are split.  For the
+// smallest a tile with a doubtful result reads its operands again (zeros by
+// cancellation among whole numbers, say), and only where they leave one does
+// it run the f32 MFMAs, for all of the tile, and take the results in doubt.
+// 2048^3, us, a kernel of f32 MFMAs only / this: normal, ReLU and softmax-tail
+// data, rows of zeros, operands of 1e-14: 166-184 / 91-100; an infinity in
+// each tile 166 / 233, subnormal operands in each 166 / 262, that is the split,
+// the second look and the second loop one after the other.
 //
 // Layout: operands go through registers (f32 loads of 4-byte alignment, one
 // step ahead of the MFMAs, two for 16-row tiles), are split there and staged
 // as three bf16 planes in the order and swizzle of the 16-bit tile family,
-// double buffered.  8
-// waves (128 x 128), two to a SIMD, so that one's splitting runs under the
-// other's MFMAs.
+// double buffered.  8 waves (128 x 128), two to a SIMD, so that one's
+// splitting runs under the other's MFMAs.
 #include "common.h"
 #include "gemm_split.h"
 #include "gemm_tile_dev.h"
@@ -65,9 +77,9 @@ __device__ __forceinline__ void split2(float x, float y, uint32_t& p1, uint32_t&
   p3 = pack_bf16x2(rx - __uint_as_float(p2 << 16), ry - __uint_as_float(p2 & 0xffff0000u));
 }
 
-constexpr float kTiny = 2.842170943040401e-14f;         // 2^-45
-constexpr float kBig = 262144.f;                           // 2^18
-constexpr float kSmallResult = 8.673617379884035e-19f;     // 2^-60
+constexpr float kWholeParts = 0x1p-100f;  // operands from here on keep all parts
+constexpr float kWholeTerms = 0x1p-96f;   // terms from here on keep all that counts
+constexpr uint32_t kInfBits = 0x7f800000u;
 
 template <int BM, int BN, int WM, int WN, int KS, bool AT, bool BT>
 __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_split_kernel(SplitArgs p) {
@@ -121,6 +133,15 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_split_kernel(SplitArgs p
   const int64_t astep = AX ? (int64_t)BK * p.lda : BK, bstep = BX ? (int64_t)BK * p.ldb : BK;
   const int NS = (K + BK - 1) / BK, whole = K / BK;  // steps; those that end inside K
 
+  uint32_t* big = reinterpret_cast<uint32_t*>(smem + 2 * STEP);  // largest magnitude of the tile's rows, then columns
+  uint32_t* small = big + BM + BN;                               // smallest nonzero one, infinity for none
+  uint32_t* flag = small + BM + BN;                              // a result in doubt; one of them finite
+  for (int i = tid; i < BM + BN; i += NW * 64) {
+    big[i] = 0;
+    small[i] = kInfBits;
+  }
+  if (tid < 2) flag[tid] = 0;
+
   // Piece w (A's, then B's) of step t; inside: t < whole.
   auto load_piece = [&](int t, int w, bool inside) {
     const bool isa = w < DA;
@@ -162,17 +183,18 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_split_kernel(SplitArgs p
   // The products of the leading parts in one accumulator, the five smaller
   // ones in another: only one rounding per 32 k at the size of the result.
   f32x4 acc[TM][TN], low[TM][TN];
-  auto clear = [&] {
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+  for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int j = 0; j < TN; ++j) acc[i][j] = low[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  };
-  clear();
+    for (int j = 0; j < TN; ++j) acc[i][j] = low[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   // The six kept products, as (part of A, part of B).
   constexpr int QA[6] = {2, 1, 0, 1, 0, 0}, QB[6] = {0, 0, 0, 1, 1, 2};
 
-  float most = 0.f;  // largest magnitude this thread has split
+  // The largest magnitude this thread has split of each piece's row (column).
+  constexpr int W = DA + DB;
+  float most[W];
+#pragma unroll
+  for (int w = 0; w < W; ++w) most[w] = 0.f;
   {
     const int af_off = frag_offset<BM, false>(wm * 16 * TM, lane);
     const int bf_off = 3 * APLANE + frag_offset<BN, false>(wn * 16 * TN, lane);
@@ -199,11 +221,11 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_split_kernel(SplitArgs p
     // Piece w of a step: its pair d of values into the three parts, and the
     // whole piece to LDS.
     u32x4 part[3];
-    auto split_pair = [&](const f32x8& v, int d) {
+    auto split_pair = [&](const f32x8& v, int w, int d) {
       const float x = d < 2 ? v.lo[2 * d] : v.hi[2 * d - 4], y = d < 2 ? v.lo[2 * d + 1] : v.hi[2 * d - 3];
       uint32_t p1, p2, p3;
       split2(x, y, p1, p2, p3);
-      most = fmaxf(most, fmaxf(fabsf(x), fabsf(y)));
+      most[w] = fmaxf(most[w], fmaxf(fabsf(x), fabsf(y)));
       part[0][d] = p1;
       part[1][d] = p2;
       part[2][d] = p3;
@@ -213,12 +235,11 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_split_kernel(SplitArgs p
 #pragma unroll
       for (int q = 0; q < 3; ++q) *reinterpret_cast<u32x4*>(at + q * (w < DA ? APLANE : BPLANE)) = part[q];
     };
-    constexpr int W = DA + DB;
     auto store = [&](int slot, const f32x8* q) {
 #pragma unroll
       for (int w = 0; w < W; ++w) {
 #pragma unroll
-        for (int d = 0; d < 4; ++d) split_pair(q[w], d);
+        for (int d = 0; d < 4; ++d) split_pair(q[w], w, d);
         put(slot, w);
       }
     };
@@ -262,7 +283,7 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_split_kernel(SplitArgs p
           if (more) {
 #pragma unroll
             for (int e = g * NP / 6; e < (g + 1) * NP / 6; ++e) {
-              split_pair(q[e / 4], e % 4);
+              split_pair(q[e / 4], e / 4, e % 4);
               if (e % 4 == 3) {
                 put(t & 1, e / 4);
                 if (kInside) q[e / 4] = load_piece(t + 3, e / 4, true);
@@ -312,84 +333,171 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_split_kernel(SplitArgs p
 #pragma unroll
     for (int j = 0; j < TN; ++j) acc[i][j] += low[i][j];
 
-  // Whether the tile has to be recomputed by f32 MFMAs (see above): bit 0 a
-  // non-finite result, 1 a small result or a big operand, 2 a tiny operand.
-  uint32_t* flags = reinterpret_cast<uint32_t*>(smem);
-  auto any = [&](uint32_t mine) {
-    __syncthreads();
-    if (tid == 0) *flags = 0;
-    __syncthreads();
-    if (mine) atomicOr(flags, mine);
-    __syncthreads();
-    const uint32_t all = *flags;
-    __syncthreads();
-    return all;
-  };
-  uint32_t seen = most > kBig ? 2u : 0u;
+  // The results to recompute by f32 MFMAs (see above), a bit each.
+  const int mloc = wm * 16 * TM + (lane & 15), nloc = wn * 16 * TN + 4 * (lane >> 4);
+  auto line = [&](int w) { return w < DA ? ax[w < DA ? w : 0] : BM + bx[w < DA ? 0 : w - DA]; };
 #pragma unroll
-  for (int i = 0; i < TM; ++i)
+  for (int w = 0; w < W; ++w) atomicMax(big + line(w), __float_as_uint(most[w]));
+  __syncthreads();
+  static_assert(TM * TN * 4 <= 32, "a bit per result");
+  const float kf = (float)K * kWholeTerms;
+  // ranged: the smallest magnitudes are known (without them: every result
+  // that is not kept for its own size, in a row and a column with a nonzero).
+  auto doubtful = [&](auto ranged) {
+    const float* bigf = reinterpret_cast<const float*>(big);
+    const float* smallf = reinterpret_cast<const float*>(small);
+    uint32_t bits = 0;
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
+    for (int j = 0; j < TN; ++j) {
+      const f32x4 bb = *reinterpret_cast<const f32x4*>(bigf + BM + nloc + 16 * j);
+      f32x4 bs = {0.f, 0.f, 0.f, 0.f};
+      if constexpr (ranged.value) bs = *reinterpret_cast<const f32x4*>(smallf + BM + nloc + 16 * j);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float m = fabsf(acc[i][j][e]);
-        seen |= !(m < __builtin_inff()) ? 1u : m < kSmallResult ? 2u : 0u;
+      for (int i = 0; i < TM; ++i) {
+        const float ab = bigf[mloc + 16 * i], as = ranged.value ? smallf[mloc + 16 * i] : 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          float m = fabsf(acc[i][j][e]);
+          if constexpr (ranged.value) asm volatile("" : "+v"(m));  // (nor from the first call to the second)
+          bool keep = m >= kf * fmaxf(1.f, fmaxf(ab, bb[e])) || fminf(ab, bb[e]) == 0.f;
+          if constexpr (ranged.value)
+            keep = keep || (as * bs[e] >= kWholeTerms && fminf(as, bs[e]) >= kWholeParts);
+          bits |= keep && m < __builtin_inff() ? 0u : 1u << (4 * (TM * j + i) + e);
+        }
       }
-  seen = any(seen);
-  if (seen == 2u) {
-    uint32_t tiny = 0;
-    for (int t = 0; t < NS; ++t) {
-      f32x8 q[DA + DB];
-      load(t, q);
+    }
+    asm volatile("" : "+v"(bits));  // (else each bit's condition is held to the end in registers of its own)
+    return bits;
+  };
+  // Whether all of this lane's results are kept for their size, by one bound.
+  auto all_large = [&] {
+    const float* bigf = reinterpret_cast<const float*>(big);
+    float most_of = 1.f;
+    f32x4 least_of = {__builtin_inff(), __builtin_inff(), __builtin_inff(), __builtin_inff()};
+    f32x4 zero = {0.f, 0.f, 0.f, 0.f};  // NaN after an infinity or a NaN
 #pragma unroll
-      for (int w = 0; w < DA + DB; ++w)
+    for (int i = 0; i < TM; ++i) most_of = fmaxf(most_of, bigf[mloc + 16 * i]);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float m = fabsf(e < 4 ? q[w].lo[e & 3] : q[w].hi[e & 3]);
-          tiny |= m < kTiny && m != 0.f ? 4u : 0u;
+    for (int j = 0; j < TN; ++j) {
+      const f32x4 bb = *reinterpret_cast<const f32x4*>(bigf + BM + nloc + 16 * j);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) most_of = fmaxf(most_of, bb[e]);
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          least_of[e] = fminf(least_of[e], fabsf(acc[i][j][e]));
+          zero[e] = __builtin_fmaf(acc[i][j][e], 0.f, zero[e]);
         }
     }
-    seen = any(tiny);
-  }
-  if (seen & 5u) {
-    // native(): f32 tiles in LDS, v_mfma_f32_16x16x4_f32; in each 32 k, lane
-    // group g feeds k = 8g + s to the s-th.
-    constexpr int LD = BK + 4;  // floats
-    float* fa = reinterpret_cast<float*>(smem);
-    float* fb = fa + BM * LD;
-    static_assert((BM + BN) * LD * 4 <= 2 * STEP, "LDS");
-    clear();
-    for (int t = 0; t < NS; ++t) {
-      f32x8 q[DA + DB];
-      load(t, q);
-      __syncthreads();
+    return zero.x + zero.y + zero.z + zero.w == 0.f &&
+           fminf(fminf(least_of.x, least_of.y), fminf(least_of.z, least_of.w)) >= kf * most_of;
+  };
+  auto in_tile = [&](uint32_t bits) {
+    if (bits) {
+      flag[0] = 1;
+      bool finite = false;
 #pragma unroll
-      for (int w = 0; w < DA + DB; ++w) {
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            finite |= (bits >> (4 * (TM * j + i) + e) & 1) && fabsf(acc[i][j][e]) < __builtin_inff();
+      if (finite) flag[1] = 1;
+    }
+    __syncthreads();
+  };
+  uint32_t redo = all_large() ? 0u : doubtful(std::false_type{});
+  in_tile(redo);
+  if (flag[1]) {
+    // Read the operands again for their smallest magnitudes, as twice their
+    // bits less one (zero: ~0).
+    uint32_t least[W];
+#pragma unroll
+    for (int w = 0; w < W; ++w) least[w] = ~0u;
+    f32x8 q[W];
+    load(0, q);
+    for (int t = 0; t < NS; ++t) {
+      f32x8 c[W];
+#pragma unroll
+      for (int w = 0; w < W; ++w) c[w] = q[w];
+      if constexpr (KS == 1) load(t + 1, q);
+#pragma unroll
+      for (int w = 0; w < W; ++w)
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          least[w] = min(least[w], 2 * __float_as_uint(e < 4 ? c[w].lo[e & 3] : c[w].hi[e & 3]) - 1);
+      if constexpr (KS > 1) load(t + 1, q);  // (its 128 k are in flight together already)
+    }
+#pragma unroll
+    for (int w = 0; w < W; ++w)
+      if (least[w] != ~0u) atomicMin(small + line(w), (least[w] >> 1) + 1);
+    __syncthreads();
+    if (tid == 0) flag[0] = 0;
+    redo = doubtful(std::true_type{});
+    __syncthreads();
+    in_tile(redo);
+  }
+  if (flag[0]) {
+    // f32 tiles in LDS (double buffered, loads a step ahead) and
+    // v_mfma_f32_16x16x4_f32; in each 32 k, lane group g feeds k = 8g + s to
+    // the s-th.  The sums go to `low`.
+    constexpr int LD = BK + 4;  // floats
+    static_assert(2 * (BM + BN) * LD * 4 <= 2 * STEP, "LDS");
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) low[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    f32x8 q[W];
+    load(0, q);
+    for (int t = 0; t < NS; ++t) {
+      float* fa = reinterpret_cast<float*>(smem) + (t & 1) * (BM + BN) * LD;
+      float* fb = fa + BM * LD;
+#pragma unroll
+      for (int w = 0; w < W; ++w) {
         float* d = w < DA ? fa + ax[w < DA ? w : 0] * LD + ak[w < DA ? w : 0]
                           : fb + bx[w < DA ? 0 : w - DA] * LD + bk[w < DA ? 0 : w - DA];
         *reinterpret_cast<f32x4*>(d) = q[w].lo;
         *reinterpret_cast<f32x4*>(d + 4) = q[w].hi;
       }
-      __syncthreads();
-      for (int s = 0; s < 8 * KS; ++s) {
-        const int k = 32 * (s >> 3) + 8 * (lane >> 4) + (s & 7);
-        float av[TM], bv[TN];
+      __syncthreads();  // step t is whole, and every wave is done with step t - 1
+      load(t + 1, q);
+#pragma unroll 1
+      for (int s = 0; s < KS; ++s) {
+        const int k = 32 * s + 8 * (lane >> 4);
+        f32x4 av[TM][2], bv[TN][2];
 #pragma unroll
-        for (int i = 0; i < TM; ++i) av[i] = fa[(wm * 16 * TM + 16 * i + (lane & 15)) * LD + k];
+        for (int h = 0; h < 2; ++h) {
 #pragma unroll
-        for (int j = 0; j < TN; ++j) bv[j] = fb[(wn * 16 * TN + 16 * j + (lane & 15)) * LD + k];
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
+          for (int i = 0; i < TM; ++i) av[i][h] = *reinterpret_cast<const f32x4*>(fa + (mloc + 16 * i) * LD + k + 4 * h);
 #pragma unroll
           for (int j = 0; j < TN; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[j], av[i], acc[i][j], 0, 0, 0);
+            bv[j][h] =
+                *reinterpret_cast<const f32x4*>(fb + (wn * 16 * TN + (lane & 15) + 16 * j) * LD + k + 4 * h);
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+#pragma unroll
+          for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+              low[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[j][e >> 2][e & 3], av[i][e >> 2][e & 3], low[i][j],
+                                                               0, 0, 0);
       }
     }
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          acc[i][j][e] = redo >> (4 * (TM * j + i) + e) & 1 ? low[i][j][e] + 0.f : acc[i][j][e];  // (-0 by underflow: +0, whatever the padding)
   }
 
   // Epilogue (C^T fragments): this lane holds row m, columns n .. n + 3.
   float* C = p.c + (int64_t)blockIdx.z * p.sc;
-  const int mrow = m0 + wm * 16 * TM + (lane & 15), ncol = n0 + wn * 16 * TN + 4 * (lane >> 4);
+  const int mrow = m0 + mloc, ncol = n0 + nloc;
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
     const int m = mrow + 16 * i;
@@ -416,7 +524,7 @@ namespace {
 
 template <int BM, int BN, int WM, int WN, int KS, bool AT, bool BT>
 hipError_t launch(const mk::SplitArgs& p, int64_t batch, hipStream_t st) {
-  constexpr size_t lds = (size_t)2 * 3 * (BM + BN) * 64 * KS;
+  constexpr size_t lds = (size_t)2 * 3 * (BM + BN) * 64 * KS + (BM + BN) * 8 + 8;
   static_assert(lds <= 160 * 1024, "LDS");
   const void* fn = (const void*)mk::gemm_split_kernel<BM, BN, WM, WN, KS, AT, BT>;
   if (lds > 64 * 1024) {
