@@ -241,10 +241,16 @@ int mk_gemm_bf16_route(const void* a, const void* b, void* c, const void* aux, i
 /* 1 when the route takes the product, else 0.  Host-only. */
 int mk_gemm_bf16_route_fits(int route, int64_t M, int64_t N, int64_t K, int epilogue, int out_f32);
 
-/* Times every route that takes the product on `stream` (warm-up and timed
- * launches: MK_GEMM_AUTOTUNE_WARMUP, default 2, and MK_GEMM_AUTOTUNE_ITERS,
- * default 5, HIP events, the median per route), records the fastest in
- * the process's route table for the current device (architecture and CU
+/* The routes that mk_gemm_bf16_autotune times for the product: those that
+ * take it, without other names of a route and without tiles whose estimated
+ * time is more than 1.4 times the best tile's.  Fills routes
+ * (MK_GEMM_ROUTE_COUNT entries) and returns their number.  Host-only. */
+int mk_gemm_bf16_autotune_routes(int64_t batch, int64_t M, int64_t N, int64_t K, int epilogue, int out_f32,
+                                 int* routes);
+
+/* Times those routes on `stream` (warm-up and timed launches:
+ * MK_GEMM_AUTOTUNE_WARMUP, default 2, and MK_GEMM_AUTOTUNE_ITERS, default 5,
+ * HIP events, the median per route), records the fastest in the process's route table for the current device (architecture and CU
  * count), shape, epilogue class and output type, and returns it in *route
  * (and its median in *us); it creates and destroys two HIP events, and
  * allocates no device memory.  c holds the product afterwards.  Not under

@@ -54,6 +54,7 @@ SIGNATURES = {
     "mk_gemm_bf16_nt": (_i32, [_p, _p, _p, _p, _i32, _i64, _i64, _i64, _i64, _p]),
     "mk_gemm_bf16_route": (_i32, [_p, _p, _p, _p, _i32, _i64, _i64, _i64, _i64, _i32, _i32, _p]),
     "mk_gemm_bf16_route_fits": (_i32, [_i32, _i64, _i64, _i64, _i32, _i32]),
+    "mk_gemm_bf16_autotune_routes": (_i32, [_i64, _i64, _i64, _i64, _i32, _i32, ctypes.POINTER(_i32)]),
     "mk_gemm_bf16_autotune": (_i32, [_p, _p, _p, _p, _i32, _i64, _i64, _i64, _i64, _i32, _p,
                                      ctypes.POINTER(_i32), ctypes.POINTER(ctypes.c_float)]),
     "mk_gemm_tuned_route": (_i32, [_i64, _i64, _i64, _i64, _i32, _i32]),
