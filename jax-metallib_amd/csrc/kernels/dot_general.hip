@@ -166,7 +166,7 @@ namespace mkg {
 bool dot_tiled(int64_t batch, int64_t M, int64_t N, int64_t K, const int64_t* sa, const int64_t* sb, DotOrder* o) {
   if (K < 16) return false;
   const int64_t top = (int64_t)1 << 30;
-  if (M > top || N > top || K > top || batch > 65535 || ((M + 15) / 16) * ((N + 63) / 64) > INT32_MAX) return false;
+  if (M > top || N > top || K > top || batch > 65535 || !tile_grid_fits(M, N, T128x128)) return false;
   bool n_contiguous = false;
   if (!operand_order(sa[1], sa[2], M, K, &o->a_t, &o->lda) ||
       !operand_order(sb[2], sb[1], N, K, &n_contiguous, &o->ldb))

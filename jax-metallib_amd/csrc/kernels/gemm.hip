@@ -740,8 +740,9 @@ int check_gemm(const char* fn, const void* a, const void* b, void* c, int64_t ba
   if (K % 8 != 0 || N % 8 != 0)
     return mkc::fail(MK_EUNSUPPORTED, "%s: needs K %% 8 == 0 and N %% 8 == 0 (got K=%lld, N=%lld)",
                      fn, (long long)K, (long long)N);
-  // Every kernel's grid (64-row tiles at the smallest, times the batch for
-  // the persistent kernel's tile count) stays below 2^31 workgroups.
+  // 64 x 64 tiles, times the batch for the persistent kernel's tile count,
+  // stay below 2^31; smaller tiles are taken only where their grid fits a
+  // launch (tile_grid_fits).
   if (M > (1 << 24) || N > (1 << 24) || K > (1 << 24) || batch > 65535 || M * K > ((int64_t)1 << 40) ||
       ((M + 63) / 64) * ((N + 63) / 64) * batch > (int64_t)INT32_MAX)
     return mkc::fail(MK_EINVAL, "%s: shape too large", fn);
@@ -801,7 +802,8 @@ bool route_fits(int route, int64_t M, int64_t N, int64_t K, int epi, int out_f32
     case MK_GEMM_ROUTE_GENERIC128:
       return simple_epi;
     default:
-      return route >= MK_GEMM_ROUTE_T16x64 && route <= MK_GEMM_ROUTE_T256x256 && simple_epi;
+      return route >= MK_GEMM_ROUTE_T16x64 && route <= MK_GEMM_ROUTE_T256x256 && simple_epi &&
+             mkg::tile_grid_fits(M, N, route - MK_GEMM_ROUTE_T16x64);
   }
 }
 

@@ -574,6 +574,8 @@ hipError_t split_launch(const SplitGemm& g, int tile, hipStream_t st) {
                                 {128, 128, 128, 1.20, 1.58, 1.39}};
     double least = 0;
     for (const Rate& r : kRates) {
+      const int64_t tiles = ((g.M + r.bm - 1) / r.bm) * ((g.N + r.bn - 1) / r.bn);
+      if (tiles * 512 > (int64_t)UINT32_MAX && r.tile != 128) continue;  // more threads than a launch has
       const double f = (double)((g.M + r.bm - 1) / r.bm) * (double)((g.N + r.bn - 1) / r.bn) * (double)g.batch / 256;
       const double t = f <= 1.0 ? r.alone + (r.full - r.alone) * f : std::max(r.full, std::ceil(f) * r.each);
       if (tile == 0 || t < least) {

@@ -31,11 +31,16 @@ struct TileGemm {
 // Tile shapes, smallest first.
 enum TileShape { T16x64 = 0, T32x64, T64x64, T128x64, T128x128, T256x256, kTileShapes };
 
+// Whether an M x N result's tiles of that shape fit a launch (2^32 threads in
+// the grid's first dimension), fed either way.
+bool tile_grid_fits(int64_t M, int64_t N, int shape);
+
 // Whether the operands' alignment lets LDS DMA feed the tiles (16-byte
 // pieces never straddle a row's end); otherwise registers do.
 bool tile_dma_ok(const TileGemm& g);
 
-// The shape the family takes for this product (tile_dma_ok included).
+// The shape the family takes for this product (tile_dma_ok included), of those
+// whose grid fits.
 int tile_pick(const TileGemm& g);
 
 // Estimated microseconds of the product in that shape, launch not counted.

@@ -491,6 +491,15 @@ constexpr double kTileOver[kTileShapes] = {0.1, 0.2, 0.3, 0.6, 1.2, 5.5};
 
 }  // namespace
 
+bool tile_grid_fits(int64_t M, int64_t N, int shape) {
+  // 256 threads a tile fed by DMA (512: 256 x 256); through registers the
+  // middle shapes are 64 x 64 tiles of 256 and the large ones 128 x 128 of 512.
+  auto fits = [&](int64_t bm, int64_t bn, int64_t threads) {
+    return ((M + bm - 1) / bm) * ((N + bn - 1) / bn) * threads <= (int64_t)UINT32_MAX;
+  };
+  return fits(kBm[shape], kBn[shape], shape == T256x256 ? 512 : 256) && (shape < T128x64 || fits(128, 128, 512));
+}
+
 bool tile_dma_ok(const TileGemm& g) {
   if (g.f16 || g.registers) return false;
   auto ok = [&](const void* q, int64_t ld, int64_t s, int64_t contiguous) {
@@ -508,16 +517,17 @@ double tile_estimate(const TileGemm& g, int shape) {
 }
 
 int tile_pick(const TileGemm& g) {
-  int best = T16x64;
-  double cost = tile_estimate(g, best);
-  for (int s = 1; s < kTileShapes; ++s) {
+  int best = -1;
+  double cost = 0;
+  for (int s = 0; s < kTileShapes; ++s) {
+    if (!tile_grid_fits(g.M, g.N, s)) continue;
     const double c = tile_estimate(g, s);
-    if (c < cost) {
+    if (best < 0 || c < cost) {
       best = s;
       cost = c;
     }
   }
-  return best;
+  return best < 0 ? T256x256 : best;
 }
 
 hipError_t tile_launch(const TileGemm& g, int shape, hipStream_t st) {
