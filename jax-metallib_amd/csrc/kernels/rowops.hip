@@ -421,7 +421,11 @@ __global__ __launch_bounds__(NT < kRowThreads ? kRowThreads : NT) void row_cache
   // exposed after the reduction.  8192^2 f32: 100.4 -> 91.6 us.  bf16 keeps
   // the load after the reduction: loaded early it costs VGPRs and waves per
   // SIMD (47.6 against 49.0 us packed, 52.9 us unpacked).
-  constexpr bool kEarly = OP == ROW_RMSNORM && GE && ALN;
+  // So do 16 vectors of 1024 threads, whose 128 registers do not hold both (64
+  // x 65536 f32 27.0 -> 12.8 us, 4096 x 40000 403 -> 259); the unaligned forms
+  // of these (and of 8 bf16 vectors) still spill: 1024 x 65535 f32 154 us
+  // against 110 aligned, 306 streamed.
+  constexpr bool kEarly = OP == ROW_RMSNORM && GE && ALN && VPT * NT <= 8 * 1024;
   u32x4 graw[kEarly ? VPT : 1];
   if constexpr (kEarly) {
 #pragma unroll
