@@ -70,6 +70,14 @@ enum { MK_QFMT_INT4_G64 = 0, MK_QFMT_INT8_PC = 1 };
 
 int64_t mk_qmatmul_workspace_bytes(int fmt, int64_t M, int64_t K, int64_t N);
 
+/* The kernels that a product of this shape runs on, its tensors aligned as
+ * an allocator gives them: the decode kernels (16 rows a pass), the mid-row
+ * kernel (qtile.hip), the many-row kernel (qgemm.hip), or a pass that writes
+ * the weights as bf16 and then the GEMM; -1 for a shape that is refused.
+ * Host-only. */
+enum { MK_QROUTE_DECODE = 0, MK_QROUTE_MID = 1, MK_QROUTE_MANY = 2, MK_QROUTE_DEQUANT = 3 };
+int mk_qmatmul_route(int fmt, int64_t M, int64_t K, int64_t N);
+
 /* 1 when a *_matmul_epilogue_bf16 call of this shape with this epilogue
  * runs, 0 when it would return an error: MK_EPI_SWIGLU_PAIRS takes the
  * dequantise-then-GEMM route only (many rows, M % 256 == 0, N % 256 == 0).

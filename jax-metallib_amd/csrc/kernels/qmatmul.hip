@@ -2153,6 +2153,15 @@ extern "C" int64_t mk_qmatmul_workspace_bytes(int fmt, int64_t M, int64_t K, int
   return std::max(p.part_bytes, base);
 }
 
+extern "C" int mk_qmatmul_route(int fmt, int64_t M, int64_t K, int64_t N) {
+  QPlan p;
+  if ((fmt != MK_QFMT_INT4_G64 && fmt != MK_QFMT_INT8_PC) || M <= 0 || K <= 0 || N <= 0 || K % 64 != 0 ||
+      !plan_base(fmt, M, K, N, &p))
+    return -1;
+  consider_qtile(fmt, M, K, N, INT64_MAX, &p);
+  return p.qt ? MK_QROUTE_MID : p.deq ? MK_QROUTE_DEQUANT : p.qg ? MK_QROUTE_MANY : MK_QROUTE_DECODE;
+}
+
 extern "C" int mk_qmatmul_epilogue_supported(int fmt, int64_t M, int64_t K, int64_t N, int epilogue) {
   if (mk_qmatmul_workspace_bytes(fmt, M, K, N) < 0) return 0;
   if (epilogue == MK_EPI_NONE || epilogue == MK_EPI_ADD || epilogue == MK_EPI_SWIGLU) return 1;

@@ -2,15 +2,14 @@
 and K split at the edges of its tiles, against the oracle, and the routes that
 stay on the older kernels.
 
-Tolerance: the kernel sums exact products (integer weights, bf16 x) in f32 and
-rounds once to bf16, 2^-8 of the value, far under the workload's rel 2e-2; the
-older kernels round the dequantised weights to bf16 too, so the two agree to
-a few 2^-8."""
+Tolerance against the oracle: the kernel sums exact products (integer weights,
+bf16 x) in f32 and rounds once to bf16, 2^-8 of the value, far under the
+workload's rel 2e-2."""
 
 import numpy as np
 import pytest
 
-from _gpu import (BF16_RTOL, assert_rel_close, dev, dev_bf16, host_bf16, host_bf16_bits, need_gpu,
+from _gpu import (BF16_RTOL, assert_rel_close, dev, dev_bf16, f32_sum_bound, host_bf16, host_bf16_bits, need_gpu,
                   torch)
 from oracle import cport, quant
 
@@ -54,33 +53,68 @@ def test_every_tile_and_split(monkeypatch, fmt, M, K, N, bm, ks):
     assert_rel_close(host_bf16(run(*args)), ref, BF16_RTOL, f"{fmt} {M}x{K}x{N} tile {bm} split {ks}")
 
 
-# Shapes the rule gives to this kernel, against the kernels it stands in for
-# (which MK_QMM_QT=0 leaves): streaming, 64-column, many-row, GEMM.
-@pytest.mark.parametrize("fmt", ["int4", "int8"])
-@pytest.mark.parametrize("M,K,N", [(100, 4096, 2048), (20, 1088, 1000), (3, 1216, 2048), (300, 1024, 1024),
-                                   (1000, 1024, 520)])
-def test_agrees_with_the_older_kernels(monkeypatch, fmt, M, K, N):
+def _route(fmt, M, K, N):
+    from mi355x import _lib
+    return _lib.lib().mk_qmatmul_route(_lib.MK_QFMT_INT4_G64 if fmt == "int4" else _lib.MK_QFMT_INT8_PC, M, K, N)
+
+
+# Shapes that the rule gives to this kernel, or leaves, against the kernels it
+# stands in for (which MK_QMM_QT=0 leaves): streaming, 64-column, many-row, GEMM.
+@pytest.mark.parametrize("fmt,M,K,N,mid", [(f, *s) for f in ("int4", "int8") for s in (
+    (100, 4096, 2048, False), (100, 2112, 2048, True), (20, 1088, 1000, True), (3, 1216, 2048, True),
+    (300, 1024, 1024, True), (1000, 1024, 520, f == "int8"))])
+def test_agrees_with_the_older_kernels(monkeypatch, fmt, M, K, N, mid):
+    """The shape's default route is what MK_QMM_QT=2 forces, bit for bit, if it
+    is this kernel, and MK_QMM_QT=0's if it is not; and the two kernels agree.
+    Each sums K products in f32 (f32_sum_bound of the terms' magnitudes, a
+    scale or two more) and rounds to bf16 (2^-9 of the value, 2^-8 together);
+    the older kernels may round each weight to bf16 before (2^-9 of its
+    term)."""
     args, run, ref = _case(fmt, M, K, N)
     print(f"[qtile] routes {fmt} M={M} K={K} N={N}", flush=True)
-    new = host_bf16(run(*args))
+    default = host_bf16_bits(run(*args))
+    monkeypatch.setenv("MK_QMM_QT", "2")
+    assert _route(fmt, M, K, N) == 1
+    forced = run(*args)
     monkeypatch.setenv("MK_QMM_QT", "0")
-    old = host_bf16(run(*args))
+    assert _route(fmt, M, K, N) != 1
+    older = run(*args)
+    monkeypatch.delenv("MK_QMM_QT")
     torch.cuda.synchronize()
+    assert (_route(fmt, M, K, N) == 1) == mid
+    assert np.array_equal(default, host_bf16_bits(forced if mid else older))
+    new, old = host_bf16(forced).astype(np.float64), host_bf16(older).astype(np.float64)
     assert_rel_close(new, ref, BF16_RTOL, f"{fmt} {M}x{K}x{N}")
     assert_rel_close(old, ref, BF16_RTOL, f"{fmt} {M}x{K}x{N} older kernel")
+    if fmt == "int4":
+        x, p, s, z = (t.cpu() for t in args)
+        q = torch.stack([p & 15, p >> 4], 1).reshape(K, N).double()
+        w = (q - z.double().repeat_interleave(64, 0)) * s.double().repeat_interleave(64, 0)
+    else:
+        x, w, s = (t.cpu().double() for t in args)
+        w = w * s
+    terms = (x.double().abs() @ w.abs()).numpy()
+    bound = 2.0 ** -8 * np.maximum(np.abs(new), np.abs(old)) + 2.0 ** -9 * terms + 2 * f32_sum_bound(terms, K + 2)
+    assert (np.abs(new - old) <= 1.01 * bound).all()
 
 
 @pytest.mark.parametrize("fmt", ["int4", "int8"])
-def test_unaligned_pointer_and_replayed_graph(fmt):
+def test_unaligned_pointer_and_replayed_graph(monkeypatch, fmt):
     """Weights 4 bytes off 16-byte alignment stay on the 64-column kernel,
-    whose loads are dwords; a captured call replays to the eager bits with
-    work between the replays."""
+    whose loads are dwords (its bits, which are not this kernel's); a captured
+    call replays to the eager bits with work between the replays."""
     args, run, ref = _case(fmt, 50, 1088, 1008)
+    assert _route(fmt, 50, 1088, 1008) == 1
     eager = host_bf16_bits(run(*args))
     flat = torch.empty(args[1].numel() + 16, dtype=args[1].dtype, device="cuda")
     w = flat[4:4 + args[1].numel()].view(args[1].shape)
     w.copy_(args[1])
-    assert_rel_close(host_bf16(run(args[0], w, *args[2:])), ref, BF16_RTOL, f"{fmt} offset weights")
+    offset = run(args[0], w, *args[2:])
+    assert_rel_close(host_bf16(offset), ref, BF16_RTOL, f"{fmt} offset weights")
+    with monkeypatch.context() as m:
+        m.setenv("MK_QMM_QT", "0")
+        older = host_bf16_bits(run(*args))
+    assert np.array_equal(host_bf16_bits(offset), older) and not np.array_equal(older, eager)
     y = torch.empty((50, 1008), dtype=torch.bfloat16, device="cuda")
     torch.cuda.synchronize()
     graph = torch.cuda.CUDAGraph()
