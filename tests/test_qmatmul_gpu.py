@@ -22,12 +22,20 @@ def _ops():
     return ops
 
 
+@pytest.fixture(params=["1", "0"], ids=["default", "older"])
+def routes(request, monkeypatch):
+    """The shape's own route, and the kernels that it has without the mid-row
+    kernel (which has most shapes of more than 16 rows)."""
+    monkeypatch.setenv("MK_QMM_QT", request.param)
+
+
 INT4_SHAPES = [
     (1, 64, 8), (16, 128, 128), (5, 256, 264), (16, 1024, 1024), (3, 512, 136),
     (17, 256, 384), (33, 192, 512), (16, 4096, 1024), (64, 2048, 896),
 ]
 
 
+@pytest.mark.usefixtures("routes")
 @pytest.mark.parametrize("M,K,N", INT4_SHAPES)
 def test_int4_g64_matches_oracle(M, K, N):
     ops = _ops()
@@ -91,6 +99,7 @@ def test_int4_g64_known_answer_all_ones():
 INT8_SHAPES = [(1, 64, 8), (16, 256, 128), (7, 512, 264), (16, 4096, 1024), (20, 320, 256)]
 
 
+@pytest.mark.usefixtures("routes")
 @pytest.mark.parametrize("M,K,N", INT8_SHAPES)
 def test_int8_pc_matches_oracle(M, K, N):
     ops = _ops()
@@ -114,7 +123,7 @@ def test_int8_pc_headline_shape():
     assert_rel_close(host_bf16(y), ref, BF16_RTOL, "int8 headline")
 
 
-# Many rows (M >= 128): the qgemm kernel (N % 128 == 0; K split in two when
+# Many rows (M >= 128) without the mid-row kernel: the qgemm kernel (N % 128 == 0; K split in two when
 # the grid has fewer than 192 tiles) or, for other N, W dequantised to bf16 in
 # the workspace and the bf16 GEMM.  The workload's M = 256 and 4096 rows at
 # reduced K, N; ragged M; K of 1, 2, 3 and 5 steps of 64 (the kernel's loop
@@ -124,6 +133,7 @@ LARGE_M_SHAPES = [(256, 4096, 2048), (4096, 512, 512), (300, 1024, 776), (512, 2
                   (200, 384, 384)]
 
 
+@pytest.mark.usefixtures("routes")
 @pytest.mark.parametrize("M,K,N", LARGE_M_SHAPES)
 def test_int4_g64_large_m_matches_oracle(M, K, N):
     ops = _ops()
@@ -136,6 +146,7 @@ def test_int4_g64_large_m_matches_oracle(M, K, N):
     assert_rel_close(host_bf16(y), ref, BF16_RTOL, f"int4 {M}x{K}x{N}")
 
 
+@pytest.mark.usefixtures("routes")
 @pytest.mark.parametrize("M,K,N", LARGE_M_SHAPES)
 def test_int8_pc_large_m_matches_oracle(M, K, N):
     ops = _ops()
@@ -150,12 +161,13 @@ def test_int8_pc_large_m_matches_oracle(M, K, N):
 
 @pytest.mark.parametrize("fmt", ["int4", "int8"])
 def test_many_row_paths_agree(monkeypatch, fmt):
-    """M = 256 through the three paths: qgemm (default), dequantise-then-GEMM
+    """M = 256 through the three older paths: qgemm, dequantise-then-GEMM
     (MK_QMM_QG_M=0) and the streaming kernels (MK_QMM_DEQ_M=0 as well).  They
     differ in the bf16 rounding of the dequantised int4 weights and in
     summation order; all meet the oracle and each other at the workload's
     bf16 tolerance."""
     ops = _ops()
+    monkeypatch.setenv("MK_QMM_QT", "0")
     rng = np.random.default_rng(77)
     M, K, N = 256, 2048, 1024
     if fmt == "int4":
@@ -183,6 +195,7 @@ def test_qgemm_kernel_many_row_tiles(monkeypatch, fmt):
     """The qgemm kernel itself over several 256-row tiles with a ragged last
     one (MK_QMM_DEQ_M=0 keeps larger M off the dequantise-then-GEMM path)."""
     ops = _ops()
+    monkeypatch.setenv("MK_QMM_QT", "0")
     monkeypatch.setenv("MK_QMM_DEQ_M", "0")
     rng = np.random.default_rng(91)
     M, K, N = 1000, 320, 256
@@ -207,6 +220,7 @@ def test_qgemm_split_k(monkeypatch, fmt, M, K, N):
     cannot change the sum), including after the unsplit call reused the
     workspace's counters."""
     ops = _ops()
+    monkeypatch.setenv("MK_QMM_QT", "0")
     rng = np.random.default_rng(5000 + M + K + N)
     if fmt == "int4":
         x, packed, s, z = quant.make_int4_case(rng, M, K, N)
@@ -240,6 +254,7 @@ def test_qgemm_exchange_in_l2_matches_device_scope(monkeypatch, fmt, M, K, N):
     outputs are bit-identical, on repeated calls too; the counters return to
     zero."""
     ops = _ops()
+    monkeypatch.setenv("MK_QMM_QT", "0")
     rng = np.random.default_rng(6000 + M + K + N)
     if fmt == "int4":
         x, packed, s, z = quant.make_int4_case(rng, M, K, N)
@@ -273,6 +288,7 @@ def test_qgemm_warp_specialised_bit_identical(monkeypatch, fmt, M, K, N):
     one step (K = 64), ragged row tiles; and within the bf16 tolerance of
     the oracle on sampled rows."""
     ops = _ops()
+    monkeypatch.setenv("MK_QMM_QT", "0")
     monkeypatch.setenv("MK_QMM_DEQ_M", "0")
     rng = np.random.default_rng(7000 + M + K + N)
     rows = np.array([0, 1, M // 2, M - 1])
@@ -352,6 +368,7 @@ def test_int4_wide_kernel_matches_oracle(monkeypatch, M, K, N, layout):
     tiles only, with 39 tiles the exchange goes through device scope)."""
     ops = _ops()
     tn, cs = WIDE_LAYOUTS[layout]
+    monkeypatch.setenv("MK_QMM_QT", "0")
     monkeypatch.setenv("MK_QMM_WIDE_TN", tn)
     monkeypatch.setenv("MK_QMM_WIDE_CS", cs)
     rng = np.random.default_rng(7 * M + K + N)
@@ -374,6 +391,7 @@ def test_int4_wide_exchange_in_l2_matches_device_scope(monkeypatch, nw, tn, M, K
     128-column tiles, one and several row blocks (2D grids), K split 2, 4
     and 8 ways (N = 2048 at 128 columns: 8)."""
     ops = _ops()
+    monkeypatch.setenv("MK_QMM_QT", "0")
     monkeypatch.setenv("MK_QMM_WIDE_NW", nw)
     monkeypatch.setenv("MK_QMM_WIDE_TN", tn)
     rng = np.random.default_rng(5 * M + K + N)
@@ -405,14 +423,16 @@ def test_int4_wide_kernel_deterministic_across_calls():
         assert np.array_equal(host_bf16_bits(ops.int4_g64_matmul(*args)), first)
 
 
+@pytest.mark.usefixtures("routes")
 def test_int4_wide_and_split_k_paths_share_a_workspace():
     """Wide-kernel calls (counters in the workspace's first 64 KB) interleaved
-    with 64-column split-K calls and the dequantise-then-GEMM path (both
-    write after the counters) through one workspace."""
+    with 64-column split-K calls, the mid-row kernel's and the
+    dequantise-then-GEMM path (all write after the counters) through one
+    workspace."""
     ops = _ops()
     rng = np.random.default_rng(23)
     for (M, K, N) in [(16, 4096, 14336), (16, 4096, 1024), (1, 8192, 8192), (5, 4096, 512),
-                      (800, 1024, 2048), (16, 4096, 14336)]:
+                      (800, 1024, 2048), (40, 4096, 1024), (16, 4096, 14336)]:
         x, packed, s, z = quant.make_int4_case(rng, M, K, N)
         y = ops.int4_g64_matmul(dev_bf16(x), dev(packed), dev_bf16(s), dev(z))
         torch.cuda.synchronize()
@@ -443,6 +463,7 @@ def test_int8_wide_kernel_matches_oracle(M, K, N, cs, monkeypatch):
     wave over all 256 columns, or waves split over two 128-column halves
     with twice the k steps) against the C oracle."""
     ops = _ops()
+    monkeypatch.setenv("MK_QMM_QT", "0")
     monkeypatch.setenv("MK_QMM_WIDE8_CS", cs)
     rng = np.random.default_rng(11 * M + K + N)
     x, w, s = quant.make_int8_case(rng, M, K, N)
@@ -491,6 +512,7 @@ SPLIT_SHAPES = [(16, 4096, 1792), (5, 2048, 1024), (20, 4096, 512), (3, 4096, 10
 def test_split_k_exchange_matches_reduce_pass(monkeypatch, fmt, M, K, N):
     ops = _ops()
     from mi355x import _lib
+    monkeypatch.setenv("MK_QMM_QT", "0")
     rng = np.random.default_rng(M + K + N + len(fmt))
     if fmt == "int4":
         x, p, s, z = quant.make_int4_case(rng, M, K, N)
