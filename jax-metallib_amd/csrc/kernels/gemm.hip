@@ -780,7 +780,6 @@ bool route_known(int route) {
          (route >= MK_GEMM_ROUTE_T16x64 && route <= MK_GEMM_ROUTE_T256x256);
 }
 
-// bt: b is B^T [N, K] (only the DMA-fed 256 x 256 kernel takes it).
 // Routes: the kernel choices of the [K, N] bf16 product (MK_GEMM_ROUTE_*).
 // Every route computes each output's k in the same order in the same MFMA,
 // so all of them give the same bits; they differ only in speed.
@@ -840,12 +839,18 @@ mkg::TileGemm tile_args(const mk::GemmArgs& p, int64_t batch, bool bt = false) {
 //     128 kernel with all of K in LDS.  MK_GEMM_SHORTK sets its largest K
 //     (default 256 on 256-multiples, 128 on other 128-multiples; 0: never).
 //   - else the tile shape whose estimated time is least (gemm_tile.hip).
+//     The estimate moves the products that do not fill 256 CUs with 256 x
+//     256 tiles to smaller ones: 2048^3 19.9 (128 x 128) against 44.6
+//     (pipelined), 1024^3 6.8 (64 x 64) against 25.0, 256 x 4096 x 4096 21.1
+//     (64 x 64) against 85.4.
 //     The pipelined 256 x 256 kernel stands in for the family's 256 x 256
-//     tiles where M and N divide, 6 % faster there (4096^3 112.7 against
-//     119.1; 128 x 128 tiles 136, hipBLASLt 110).  The estimate moves the
-//     products that do not fill 256 CUs with such tiles to smaller ones:
-//     2048^3 24.8 (128 x 128) against 45 (pipelined), 1024^3 7.9 (64 x 64)
-//     against 25, 256 x 4096 x 4096 20.3 (64 x 64) against 79.
+//     tiles where M and N divide: 4096^2 x 512 21.0 against 21.9, from K =
+//     1024 within 2 % either way (4096^3 105.1 / 104.1, 8192 x 2048 x 8192
+//     208.9 / 204.8).  It is kept where its estimate is up to 6 % above that
+//     of 128 x 128 tiles (0.94), which several rounds of such tiles do not
+//     bear out: 16 x 1024 x 768 x 8192 228 against 272, 8 x 768 x 1536 x 4096
+//     111 / 124, 6144 x 1536 x 2048 49.8 / 54.5; at K = 512 the same, or 4 x
+//     3072 x 6144 x 512 103 / 100.
 int default_route(const mkg::TileGemm& g) {
   const int64_t batch = g.batch, M = g.M, N = g.N, K = g.K;
   const int epi = g.epi, out_f32 = g.out_f32 ? 1 : 0;
@@ -980,7 +985,8 @@ int run_gemm_bf16(const char* fn, const void* a, const void* b, void* c, const v
   hipStream_t st = static_cast<hipStream_t>(stream);
   hipError_t e;
   const mkg::TileGemm tg = tile_args(p, batch, bt);
-  // B^T: the smaller tiles where the estimate prefers them, as for [K, N].
+  // B^T: the smaller tiles where the estimate prefers them, by the rule for
+  // [K, N] (default_route); else the 256 x 256 kernels that read B^T.
   const int bt_shape = bt && epi != MK_EPI_SWIGLU_PAIRS && !tg.registers ? mkg::tile_pick(tg) : mkg::T256x256;
   if (bt && bt_shape != mkg::T256x256 &&
       mkg::tile_estimate(tg, bt_shape) < 0.94 * mkg::tile_estimate(tg, mkg::T256x256)) {

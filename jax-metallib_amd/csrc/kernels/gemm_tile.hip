@@ -447,8 +447,8 @@ hipError_t launch_dma(const mk::TileArgs& p, int64_t batch, int shape, hipStream
     case T128x128:
       // A workgroup alone on its CU needs two steps in flight (96 KB of
       // LDS); with more tiles than CUs two workgroups of one step each
-      // cover for one another.  Two steps / one: 2048^3 (256 tiles) 24.8 /
-      // 29.2 us, 2000 x 3000 x 2048 (384) 41.7 / 33.2, 4096^3 163 / 136.
+      // cover for one another.  Two steps / one: 2048^3 (256 tiles) 19.8 /
+      // 24.9 us, 2000 x 3000 x 2048 (384) 35.2 / 30.0, 4096^3 151 / 133.
       if ((int64_t)((p.M + 127) / 128) * ((p.N + 127) / 128) * batch <= kCus)
         return launch<128, 128, 2, 2, 2, 3, AT, BT, false, true>(p, batch, st);
       return launch<128, 128, 2, 2, 2, 2, AT, BT, false, true>(p, batch, st);
@@ -456,7 +456,9 @@ hipError_t launch_dma(const mk::TileArgs& p, int64_t batch, int shape, hipStream
   }
 }
 
-// Fed through registers: three shapes.
+// Fed through registers: three shapes.  f16 has these only: such products come
+// from dot_general alone, and the DMA-fed instances, most of this file's code,
+// are bf16's.
 template <bool AT, bool BT, bool F16>
 hipError_t launch_reg(const mk::TileArgs& p, int64_t batch, int shape, hipStream_t st) {
   switch (shape) {
