@@ -332,8 +332,8 @@ CHAIN6 = [("LOAD", 0, 0, 0, 0, 0.0), ("CONST", 1, 0, 0, 0, 1.5), ("MUL", 2, 0, 1
           ("LOG1P", 5, 4, 0, 0, 0.0), ("MAX", 6, 5, 0, 0, 0.0), ("CONST", 1, 0, 0, 0, 0.0),
           ("CMP_GT", 7, 0, 1, 0, 0.0), ("SELECT", 8, 7, 6, 3, 0.0)]
 
-PROFILE_KINDS = ("int4", "int8", "gemm", "gemm_f32", "qgemm", "qgemm8", "int4_m1", "int8_m1", "int4_shard",
-                 "int8_shard", "bmm", "dequant4096", "dequant4096_8", "attention", "softmax_f32", "softmax_bf16",
+PROFILE_KINDS = ("int4", "int8", "gemm", "gemm_f32", "gemm_16", "gemm_1000", "gemm_2000", "qtile", "qtile8",
+                 "qtile8_100", "qgemm", "int4_m1", "int8_m1", "int4_shard", "int8_shard", "bmm", "dequant4096", "dequant4096_8", "attention", "softmax_f32", "softmax_bf16",
                  "rmsnorm_f32", "rmsnorm_bf16", "argmax_f32", "argmax_bf16", "chain6_f32", "chain6_bf16")
 
 
@@ -347,28 +347,30 @@ def _profile_case(torch, ops, kind):
 
     rng = np.random.default_rng(0)
     g = torch.Generator(device="cuda").manual_seed(0)
-    quant = {"int4": (16, 14336), "qgemm": (256, 14336), "int4_m1": (1, 14336), "int4_shard": (16, 1792),
-             "dequant4096": (4096, 14336)}
+    quant = {"int4": (16, 14336), "qtile": (256, 14336), "qgemm": (512, 14336), "int4_m1": (1, 14336),
+             "int4_shard": (16, 1792), "dequant4096": (4096, 14336)}
     if kind in quant:
         M, N = quant[kind]
         x, packed, s, z = synthetic.int4_case(rng, M, 4096, N)
         xd, wd, sd, zd = bf(x), torch.from_numpy(packed).cuda(), bf(s), torch.from_numpy(z).cuda()
         yd = torch.empty((M, N), dtype=torch.bfloat16, device="cuda")
         return lambda: ops.int4_g64_matmul(xd, wd, sd, zd, out=yd)
-    if kind in ("int8", "int8_m1", "int8_shard", "qgemm8", "dequant4096_8"):
-        M, N = {"int8": (16, 14336), "int8_m1": (1, 14336), "int8_shard": (16, 1792), "qgemm8": (256, 14336),
-                "dequant4096_8": (4096, 14336)}[kind]
+    if kind in ("int8", "int8_m1", "int8_shard", "qtile8", "qtile8_100", "dequant4096_8"):
+        M, N = {"int8": (16, 14336), "int8_m1": (1, 14336), "int8_shard": (16, 1792), "qtile8": (256, 14336),
+                "qtile8_100": (100, 14336), "dequant4096_8": (4096, 14336)}[kind]
         x, w8, s8 = synthetic.int8_case(rng, M, 4096, N)
         xd, wd, sd = bf(x), torch.from_numpy(w8).cuda(), torch.from_numpy(s8).cuda()
         yd = torch.empty((M, N), dtype=torch.bfloat16, device="cuda")
         return lambda: ops.int8_pc_matmul(xd, wd, sd, out=yd)
-    if kind in ("gemm", "bmm"):
-        batch, M, N, K = (1, 4096, 4096, 4096) if kind == "gemm" else (16, 2048, 2048, 128)
+    gemms = {"gemm": (1, 4096, 4096, 4096), "bmm": (16, 2048, 2048, 128), "gemm_16": (1, 16, 14336, 4096),
+             "gemm_1000": (1, 1000, 14336, 4096), "gemm_2000": (1, 2000, 3000, 2048)}
+    if kind in gemms:
+        batch, M, N, K = gemms[kind]
         sc = 1.0 / np.sqrt(np.sqrt(K))
         a = (torch.randn((batch, M, K), device="cuda", generator=g) * sc).to(torch.bfloat16)
         b = (torch.randn((batch, K, N), device="cuda", generator=g) * sc).to(torch.bfloat16)
         c = torch.empty((batch, M, N), dtype=torch.bfloat16, device="cuda")
-        if kind == "gemm":
+        if batch == 1:
             a, b, c = a[0], b[0], c[0]
         return lambda: ops.gemm_bf16(a, b, out=c)
     if kind == "gemm_f32":
@@ -898,9 +900,7 @@ def main():
                                           "unit": "TFLOP/s", "frac": round(tf / BF16_PEAK_TFLOPS, 4),
                                           "traffic": None}}
                     if M == 256:
-                        qt, qn = traffic_from_profiles(
-                            "qgemm_ws_kernel_M256_K4096_N14336" if fmt == "int4"
-                            else "qgemm_ws_kernel_int8_M256_K4096_N14336")
+                        qt, qn = traffic_from_profiles(f"qtile_kernel_{fmt}_M256_K4096_N14336")
                         entry["roofline"].update({"traffic": qt, "traffic_note": qn})
                     if M == 4096:
                         # The route's GEMM (the MFMA roofline above; same
@@ -965,7 +965,7 @@ def main():
             secondary["bf16_bmm_16x2048x128x2048"]["cpu_baseline"] = cpu_baseline_bmm(args.cpu_row_seconds)
         rf = bench_gemm_f32(torch, ops, max(50, args.steps // 20), 5)
         log(f"[bench] f32 gemm 2048^3: {rf['sec_per_call'] * 1e6:.1f} us, {rf['tflops']:.1f} TFLOP/s")
-        ft, fnote = traffic_from_profiles("gemm_f32_kernel_2048")
+        ft, fnote = traffic_from_profiles("gemm_split_kernel_2048")
         secondary["f32_gemm_2048"] = {
             "value": round(rf["tflops"], 2), "unit": "TFLOP/s", "us_per_call": round(rf["sec_per_call"] * 1e6, 3),
             "roofline": {"bound": "mfma", "achieved": round(rf["tflops"], 2), "peak": 157.3,
