@@ -333,8 +333,9 @@ CHAIN6 = [("LOAD", 0, 0, 0, 0, 0.0), ("CONST", 1, 0, 0, 0, 1.5), ("MUL", 2, 0, 1
           ("CMP_GT", 7, 0, 1, 0, 0.0), ("SELECT", 8, 7, 6, 3, 0.0)]
 
 PROFILE_KINDS = ("int4", "int8", "gemm", "gemm_f32", "gemm_16", "gemm_1000", "gemm_2000", "qtile", "qtile8",
-                 "qtile8_100", "qgemm", "int4_m1", "int8_m1", "int4_shard", "int8_shard", "bmm", "dequant4096", "dequant4096_8", "attention", "softmax_f32", "softmax_bf16",
-                 "rmsnorm_f32", "rmsnorm_bf16", "argmax_f32", "argmax_bf16", "chain6_f32", "chain6_bf16")
+                 "qtile8_100", "qgemm", "int4_m1", "int8_m1", "int4_shard", "int8_shard", "bmm", "dequant4096",
+                 "dequant4096_8", "attention", "softmax_f32", "softmax_bf16", "rmsnorm_f32", "rmsnorm_bf16",
+                 "argmax_f32", "argmax_bf16", "chain6_f32", "chain6_bf16")
 
 
 def _profile_case(torch, ops, kind):
